@@ -103,7 +103,8 @@ int qmm_matvec(int type, const void *w, const void *xq, float *dst, int64_t ldd,
  * reference's few-rows policy (quantized/cuda.rs:775-839): the decode
  * kernels up to qmm_matvec_max_rows() rows; for Q4_K and Q6_K the few-row
  * int8 matrix-core kernels from 4 rows on weights of 2 MiB or more and for
- * 9-32 rows, then the int8 matrix-core GEMMs from 33 rows; for Q8_0, IQ4_NL
+ * 9-16 rows, the exact short-batch kernel for 17-128 rows, then the int8
+ * matrix-core GEMMs; for Q8_0, IQ4_NL
  * and MXFP4 the int8 matrix-core GEMM from 9 rows. Nothing is allocated.
  * The SWARMLLM_QMATMUL_MMQ switches below move these lines. Replaces
  * swarm_mmq_matmul's launch step (mmq_entry.cu:162-203), which multiplies
@@ -137,7 +138,7 @@ int qmm_mmq_captured(void);
  * feed the matrix cores a rounded product of a code and its sub-block scale
  * (normalised error up to about 1e-3, inside the 2e-3 bound): the
  * single-pass Q4_K and Q6_K GEMMs (from 129 rows) and the few-row Q6_K
- * kernel's single-product form (k >= 2048, from the few-rows line to 32 rows), so a product's bits
+ * kernel's single-product form (k >= 2048, from the few-rows line to 16 rows), so a product's bits
  * can depend on the row count of its batch (1-2 rows are always exact). With
  * it every row count sums exact int32 products, at the exact kernels' speed.
  * qmm_exact_forms: 1 when the switch is on. */
@@ -180,10 +181,11 @@ int qmm_accumulate_in_f32(int type);
  * *need is set to the workspace bytes the launch will want; with
  * launch != 0 the product is enqueued, and QMM_WORKSPACE_TOO_SMALL is
  * returned (nothing enqueued) when workspace_bytes is less than the
- * quantized activation. For a single-pass Q4_K GEMM whose tiles fill at
- * most half the CUs, *need also counts the slots of a K split (the product
- * cut into 2 or 4 parts along K, added in part order); with a workspace that
- * holds the activation but not those slots the product runs uncut.
+ * quantized activation. For a single-pass GEMM whose tiles fill at
+ * most half the CUs, and for Q4_K and Q6_K at 17-128 rows, *need also counts
+ * the slots of a K split (the product cut into parts along K, added in part
+ * order); with a workspace that holds the activation but not those slots the
+ * product runs uncut (at 17-128 rows with the same bits).
  * Replaces the plan/launch pair of swarm_mmq_matmul (mmq_entry.cu:162-203). */
 int qmm_forward(int type, const void *w, const float *x, int64_t x_stride, float *dst, int64_t ldd,
                 void *workspace, size_t workspace_bytes, size_t *need, int64_t k, int64_t n, int64_t rows,
@@ -215,8 +217,8 @@ size_t qmm_forward_noalloc_max_bytes(void);
  * rows the products run as one launch per 4 weights, each quantizing the
  * activation in LDS (workspace unused); otherwise the activation is
  * quantized once into the workspace and each weight's product reads it, the
- * weights the few-row matrix-core kernels or the single-pass Q4_K GEMM take
- * sharing one launch per 4 (each weight's K split as its own forward would
+ * weights the few-row and short-batch matrix-core kernels or the single-pass
+ * GEMMs take sharing one launch per 4 (each weight's K split as its own forward would
  * choose, so results equal qmm_forward's bit for bit). Plan (launch == 0) and
  * launch as qmm_forward. Replaces QMatMul::forward_shared with the CUDA
  * arm's shared activation (quantized/mod.rs:1221-1263,

@@ -1,0 +1,560 @@
+// gemm_kq_mid.hip — Q4_K and Q6_K products of 17 to 128 activation rows on
+// the int8 matrix cores of gfx950: short prompts, large decode batches.
+//
+// dst[m][n] = sum over super-blocks of candle's Q4_K / Q6_K x Q8_K vec_dot
+// (vendor/candle/candle-core/src/quantized/k_quants.rs:2031-2111, 2598-2655)
+// against the activation quantized as the reference quantizes it
+// (BlockQ8K::from_float, :2882-2927): per-256 scale dy, int8 codes y, code
+// sums S of 16 values.
+//
+// Exact integers. Q4_K: sc q (10 bits) enters as two int8 operands, sc =
+// 8 sh + sl, sh q and sl q <= 105 (one packed 16-bit multiply makes four of
+// them: the products stay inside their bytes), T = 8 T_h + T_l; the min sums
+// Tm = sum_j m_j S_j run on one f16 product of small integers (S of 16 values
+// and m_j are exact in f16, every sum stays below 2^24). Q6_K: p = sc (q - 32)
+// (14 bits) enters as the high byte h and the low byte minus 128, l, of
+// 4p + 128: 256 T_h + T_l = 4 sum p y. The f32 epilogue of a super-block is
+// acc += dy (d T - dmin Tm), Q6_K acc += dy (d/4 T).
+//
+// What bounds these products is getting the weight to enough CUs: at 17-128
+// rows a weight's bytes (33 MB for 14336 x 4096: 7 us at the 4.8 TB/s a copy
+// reaches) and its MFMAs (MT row tiles x 17 x 32 cycles a super-block of 32
+// weight rows) are both a few microseconds, while a tile that walks all of K
+// alone takes 2 us a super-block (the tiled GEMMs, uncut, at 77 rows: q, k, v
+// and o 36 us each, gate and up 39 each, the Q6_K down 110). So K is cut: a workgroup takes
+// 32 kNW weight rows, ALL activation rows (MT tiles of 32, so a weight byte is
+// read and expanded once) and one of S ranges of super-blocks; its partial
+// goes to a slot and a second launch adds the slots in split order.
+//
+// Workgroup: kNW waves, each 32 weight rows x MT tiles of
+// v_mfma_i32_32x32x32_i8 (one MFMA per 32-value group, tile and operand).
+//   - The activation codes of a super-block (32 MT rows x 256 B, pieces
+//     XOR-swizzled by row) reach LDS by direct copies, one super-block ahead,
+//     double-buffered; the code sums (as f16) and dy through registers.
+//   - A wave's raw weight bytes (32 rows' blocks as their aligned 16-byte
+//     pieces) are loaded one super-block ahead into registers, consecutive
+//     lanes on consecutive pieces, and written to the wave's own LDS slot
+//     when the current super-block is done; lanes read their row back.
+//     Q4_K's rows lie 144 bytes apart there, Q6_K's 240 (both spread 16 rows
+//     over the banks).
+// Rows past M and weight rows past N are read as the last row (valid memory);
+// their outputs are never stored.
+//
+// Measured at 77 rows (an 8B layer, slots added in): q + k + v 24 us, o 19.5,
+// gate + up with its GLU 46, down 35; at 21 rows 15 / 13 / 28 / 26 (the
+// two-row-tile few-row kernels before: 13 / 9 / 54 / 25). At 21 rows gate + up
+// reads HBM at 4.9 TB/s, 1.5 x its weight bytes (the 64-byte sector at each
+// 144-byte block's edges is fetched twice); at 77 the vector unit is busy 41%
+// and the matrix cores 30% of the time. The weight loads are nontemporal:
+// plain ones took 50 us at 21 rows, 62 at 77. A second super-block of
+// weights in flight changed nothing.
+//
+// A product's bits do not depend on the workspace: without room for the
+// slots one workgroup computes a tile's splits one after another and adds
+// each to dst, the same sums in the same order.
+#include "lds_copy.h"
+#include "mv_common.h"
+#include "qmm_device.h"
+#include "qmm_launch.h"
+
+namespace qmm {
+
+namespace {
+
+typedef int i4v __attribute__((ext_vector_type(4)));
+typedef int i16v __attribute__((ext_vector_type(16)));
+typedef float f16v __attribute__((ext_vector_type(16)));
+typedef float f4v __attribute__((ext_vector_type(4)));
+typedef _Float16 h8 __attribute__((ext_vector_type(8)));
+typedef _Float16 h2v __attribute__((ext_vector_type(2)));
+typedef unsigned short u16x2 __attribute__((ext_vector_type(2)));
+
+__device__ __forceinline__ uint32_t pkmul(uint32_t a, uint32_t b) {
+  return __builtin_bit_cast(uint32_t, (u16x2)(__builtin_bit_cast(u16x2, a) * __builtin_bit_cast(u16x2, b)));
+}
+__device__ __forceinline__ uint32_t pkmad(uint32_t a, uint32_t b, uint32_t c) {
+  return __builtin_bit_cast(uint32_t, (u16x2)(__builtin_bit_cast(u16x2, a) * __builtin_bit_cast(u16x2, b) +
+                                               __builtin_bit_cast(u16x2, c)));
+}
+
+struct MidArgs {
+  const void* w[kMaxTargets];
+  float* dst[kMaxTargets];
+  int64_t ldd[kMaxTargets];
+  int64_t n[kMaxTargets];
+  int unit_end[kMaxTargets];      // workgroups of weights 0..t
+  int splits[kMaxTargets];        // K ranges of weight t
+  int64_t part_off[kMaxTargets];  // its slots in `part` (floats): [split][M][n]
+  const int8_t* yq;
+  const float* yd;
+  const int16_t* ybs;
+  float* part;  // null: uncut, a workgroup walks a tile's splits in turn
+  int M, nsb, remap;
+};
+
+template <int FMT>
+struct MidFmt {
+  static constexpr bool kQ6 = FMT == T_Q6_K;
+  static constexpr int kBlock = kQ6 ? 210 : 144;
+  static constexpr int kPieces = kQ6 ? 14 : 9;              // aligned pieces around a row's block
+  static constexpr int kStride = kQ6 ? 240 : 144;           // LDS bytes a row
+  static constexpr int kLoads = (32 * kPieces + 63) / 64;   // a wave's 64-lane loads a super-block
+  static constexpr int kSlot = 32 * kStride + (kQ6 ? 16 : 0);
+};
+
+// kWide (97-128 rows): one set of integer accumulators, the high operand's
+// products first, then shifted, then the low operand's; the two sets of four
+// row tiles and their f32 sums would leave no registers for the rest.
+template <int FMT, int MT, int kNW, bool kWide>
+__global__ __launch_bounds__(64 * kNW, 2) void gemm_kq_mid_kernel(const MidArgs a) {
+  using F = MidFmt<FMT>;
+  constexpr bool Q6 = F::kQ6;
+  constexpr int kRows = 32 * MT, BN = 32 * kNW, kThreads = 64 * kNW;
+  constexpr int kACopies = 8 * MT / kNW;  // a wave's 1 KB activation copies a super-block
+  static_assert(8 * MT % kNW == 0 && 2 * kRows <= kThreads, "copy shapes");
+  __shared__ __attribute__((aligned(1024))) int8_t s_a[2][kRows * 256];
+  __shared__ __attribute__((aligned(16))) uint8_t s_w[kNW][F::kSlot];
+  __shared__ __attribute__((aligned(16))) _Float16 s_bs[2][Q6 ? 1 : kRows][16];
+  __shared__ __attribute__((aligned(16))) float s_dy[2][kRows];
+
+  const int tid = threadIdx.x;
+  const int lane = tid & 63;
+  const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int h = lane >> 5, r32 = lane & 31;
+
+  const int total = (int)gridDim.x;
+  const int b = (int)blockIdx.x;
+  const int idx = a.remap ? (b & 7) * (total >> 3) + (b >> 3) : b;
+  const int t = idx < a.unit_end[0] ? 0 : idx < a.unit_end[1] ? 1 : idx < a.unit_end[2] ? 2 : 3;
+  auto pick = [&](const auto& arr) { return t == 0 ? arr[0] : t == 1 ? arr[1] : t == 2 ? arr[2] : arr[3]; };
+  const int loc = idx - (t == 0 ? 0 : t == 1 ? a.unit_end[0] : t == 2 ? a.unit_end[1] : a.unit_end[2]);
+  const int64_t N = pick(a.n);
+  const int S = pick(a.splits);
+  const int nsb = a.nsb, M = a.M;
+  const int ctiles = (int)((N + BN - 1) / BN);
+  const bool cut = a.part != nullptr;
+  const int ct = cut ? loc % ctiles : loc;
+  const int s0 = cut ? loc / ctiles : 0, s1 = cut ? s0 + 1 : S;
+  const uint8_t* __restrict__ W = (const uint8_t*)pick(a.w);
+  const int8_t* __restrict__ yq = a.yq;
+  const float* __restrict__ yd = a.yd;
+  const int16_t* __restrict__ ybs = a.ybs;
+  const int64_t n0 = (int64_t)ct * BN;
+  const uint32_t K = (uint32_t)nsb * 256u;
+  const uint32_t rowbytes = (uint32_t)nsb * F::kBlock;
+
+  // activation copies: copy i moves rows 4i .. 4i+3; lane L writes row
+  // 4i + L/16 at piece position L%16, which holds code piece (L%16) ^ (row & 15)
+  uint32_t aoff[kACopies];
+#pragma unroll
+  for (int u = 0; u < kACopies; u++) {
+    const int row = 4 * (wv + kNW * u) + (lane >> 4);
+    aoff[u] = (uint32_t)(row < M ? row : M - 1) * K + 16u * (((uint32_t)lane & 15u) ^ ((uint32_t)row & 15u));
+  }
+  auto copy_a = [&](int sb, int buf) {
+#pragma unroll
+    for (int u = 0; u < kACopies; u++)
+      dma16(yq + 256 * (int64_t)sb, aoff[u], lds_addr(&s_a[buf][1024 * (wv + kNW * u)]));
+  };
+  // weight pieces: piece f = 64u + lane of the wave's 32 rows (row f / kPieces)
+  uint32_t woff[F::kLoads];
+#pragma unroll
+  for (int u = 0; u < F::kLoads; u++) {
+    uint32_t f = 64u * (uint32_t)u + (uint32_t)lane;
+    if (f > 32u * F::kPieces - 1u) f = 32u * F::kPieces - 1u;
+    const uint32_t row = f / (uint32_t)F::kPieces;
+    const int64_t gr = n0 + 32 * wv + row < N ? n0 + 32 * wv + row : N - 1;
+    woff[u] = (uint32_t)gr * rowbytes + 16u * (f - (uint32_t)F::kPieces * row);
+  }
+  uint4 wr[F::kLoads];
+  auto load_w = [&](int sb) {
+#pragma unroll
+    for (int u = 0; u < F::kLoads; u++) {
+      if constexpr (Q6)
+        wr[u] = ld_stream16(W + ((woff[u] + 210u * (uint32_t)sb) & ~15u));
+      else
+        wr[u] = ld_stream16(W + 144 * (int64_t)sb + woff[u]);
+    }
+  };
+  auto store_w = [&]() {
+#pragma unroll
+    for (int u = 0; u < F::kLoads; u++) {
+      uint32_t f = 64u * (uint32_t)u + (uint32_t)lane;
+      if (32 * F::kPieces % 64 != 0 && u == F::kLoads - 1 && f > 32u * F::kPieces - 1u) f = 32u * F::kPieces - 1u;
+      if constexpr (Q6) f += f / (uint32_t)F::kPieces;  // 15 pieces a row in LDS
+      *(uint4*)&s_w[wv][16u * f] = wr[u];
+    }
+  };
+  // code sums and dy: thread -> (row, half) and row, threads past them
+  // repeating the first ones' (no branch in a step)
+  const int bt = tid % (2 * kRows), dt = tid % kRows;
+  const int brow = (bt >> 1) < M ? bt >> 1 : M - 1;
+  const int drow = dt < M ? dt : M - 1;
+  uint4 bs = {};
+  float dyr = 0.0f;
+  auto load_rows = [&](int sb) {
+    if (!Q6) bs = *(const uint4*)(ybs + (int64_t)brow * (K / 16) + 16 * sb + 8 * (bt & 1));
+    dyr = yd[(int64_t)drow * nsb + sb];
+  };
+  auto store_rows = [&](int buf) {
+    if (!Q6) {
+      const uint32_t w4[4] = {bs.x, bs.y, bs.z, bs.w};
+      h8 v;
+#pragma unroll
+      for (int i = 0; i < 4; i++) {
+        v[2 * i] = (_Float16)(int16_t)(w4[i] & 0xFFFFu);
+        v[2 * i + 1] = (_Float16)(int16_t)(w4[i] >> 16);
+      }
+      *(h8*)&s_bs[buf][bt >> 1][8 * (bt & 1)] = v;
+    }
+    s_dy[buf][dt] = dyr;
+  };
+
+  // the lane's weight row in its wave's slot (Q6_K: its block starts at byte
+  // (wbase + 210 sb) mod 16 of it), and its activation row's operand address
+  const uint8_t* wrow = &s_w[wv][r32 * F::kStride];
+  const int64_t grow = n0 + 32 * wv + r32 < N ? n0 + 32 * wv + r32 : N - 1;
+  const uint32_t wbase = (uint32_t)grow * rowbytes;
+  const uint32_t fa0 = 256u * (uint32_t)r32 + 16u * ((uint32_t)h ^ ((uint32_t)r32 & 15u));
+
+  f16v acc[MT];
+  float* __restrict__ dst = pick(a.dst);
+  const int64_t ldd = pick(a.ldd);
+  const int64_t col = n0 + 32 * wv + r32;
+
+  for (int s = s0; s < s1; s++) {
+    const int sb0 = s * nsb / S, sb1 = (s + 1) * nsb / S;
+#pragma unroll
+    for (int m = 0; m < MT; m++)
+#pragma unroll
+      for (int i = 0; i < 16; i++) acc[m][i] = 0.0f;
+    copy_a(sb0, 0);
+    load_w(sb0);
+    load_rows(sb0);
+    store_w();
+    store_rows(0);
+    __builtin_amdgcn_s_waitcnt(0);
+    __syncthreads();
+
+    for (int sb = sb0; sb < sb1; sb++) {
+      const int cur = (sb - sb0) & 1;
+      const int nx = sb + 1 < sb1 ? sb + 1 : sb;  // past the last super-block, the last one's again
+      copy_a(nx, cur ^ 1);
+      load_w(nx);
+      load_rows(nx);
+
+      const int8_t* sa = s_a[cur];
+      i16v th[MT], tl[MT];
+      h8 mb = {};
+      float d = 0.0f, dmin = 0.0f;
+      auto afrag = [&](int j, int m) -> i4v { return *(const i4v*)(sa + (fa0 ^ (32u * (uint32_t)j)) + 8192 * m); };
+      // one group's operands against every row tile; which: 1 high, 2 low, 3 both
+      auto mul = [&](int j, int which, const i4v& bh, const i4v& bl) {
+        const i16v zero = {};
+#pragma unroll
+        for (int m = 0; m < MT; m++) {
+          const i4v af = afrag(j, m);
+          if (which & 1) th[m] = __builtin_amdgcn_mfma_i32_32x32x32_i8(af, bh, j == 0 ? zero : th[m], 0, 0, 0);
+          if (which & 2)
+            tl[m] = __builtin_amdgcn_mfma_i32_32x32x32_i8(af, bl, j == 0 && !kWide ? zero : tl[m], 0, 0, 0);
+        }
+      };
+      auto widen = [&]() {  // kWide: the high products scaled, the low ones added to them
+#pragma unroll
+        for (int m = 0; m < MT; m++)
+#pragma unroll
+          for (int i = 0; i < 16; i++) tl[m][i] = (int)((uint32_t)th[m][i] << (Q6 ? 8 : 3));
+      };
+      if constexpr (!Q6) {
+        const uint4 hdr = *(const uint4*)wrow;
+        d = h2f((uint16_t)(hdr.x & 0xFFFFu));
+        dmin = h2f((uint16_t)(hdr.x >> 16));
+        // 6-bit scales and mins (get_scale_min_k4, vendor/candle/candle-core/src/quantized/utils.rs:50-60)
+        const uint32_t sc[2] = {hdr.y & 0x3f3f3f3fu, (hdr.w & 0x0f0f0f0fu) | (((hdr.y >> 6) & 0x03030303u) << 4)};
+        const uint32_t mn = h ? ((hdr.w >> 4) & 0x0f0f0f0fu) | (((hdr.z >> 6) & 0x03030303u) << 4)
+                              : hdr.z & 0x3f3f3f3fu;
+        const uint32_t sl[2] = {sc[0] & 0x07070707u, sc[1] & 0x07070707u};
+        const uint32_t sh[2] = {(sc[0] >> 3) & 0x07070707u, (sc[1] >> 3) & 0x07070707u};
+        // Tm: K slots 8h .. 8h+7 hold the 16-value sums 8h .. and m_j twice each
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+          // 1024 + m as f16 bits twice, minus 1024: exact
+          const h2v v = __builtin_bit_cast(h2v, __builtin_amdgcn_perm(0x64646464u, mn, 0x04000400u + 0x00010001u * i)) -
+                        (h2v){(_Float16)1024.0f, (_Float16)1024.0f};
+          mb[2 * i] = v[0];
+          mb[2 * i + 1] = v[1];
+        }
+        auto sweep = [&](int which) {
+#pragma unroll
+          for (int c = 0; c < 4; c++) {
+            const uint4 raw = *(const uint4*)(wrow + 16 + 32 * c + 16 * h);
+            const uint32_t rw[4] = {raw.x, raw.y, raw.z, raw.w};
+#pragma unroll
+            for (int p = 0; p < 2; p++) {
+              const int j = 2 * c + p;
+              const uint32_t sel = 0x0C000C00u + 0x00010001u * (uint32_t)(j & 3);
+              const uint32_t hj = __builtin_amdgcn_perm(0u, sh[j >> 2], sel);
+              const uint32_t lj = __builtin_amdgcn_perm(0u, sl[j >> 2], sel);
+              i4v bh = {}, bl = {};
+#pragma unroll
+              for (int e = 0; e < 4; e++) {
+                const uint32_t q = (p ? rw[e] >> 4 : rw[e]) & 0x0F0F0F0Fu;
+                if (which & 1) bh[e] = (int)pkmul(q, hj);
+                if (which & 2) bl[e] = (int)pkmul(q, lj);
+              }
+              mul(j, which, bh, bl);
+              if constexpr (MT > 2) __builtin_amdgcn_sched_barrier(0);
+            }
+          }
+        };
+        if constexpr (kWide) {
+          sweep(1);
+          widen();
+          sweep(2);
+        } else {
+          sweep(3);
+        }
+      } else {
+        const int o = (int)((wbase + 210u * (uint32_t)sb) & 15u);
+        uint32_t scw[4];
+        lds_words<4>(wrow, o + 192, scw);
+        d = 0.25f * h2f((uint16_t)lds_u16(wrow, o + 208));
+        auto sweep = [&](int which) {
+#pragma unroll
+          for (int hf = 0; hf < 2; hf++) {
+            uint32_t ql[2][4], qh[4];
+            lds_words<4>(wrow, o + 64 * hf + 16 * h, ql[0]);
+            lds_words<4>(wrow, o + 64 * hf + 32 + 16 * h, ql[1]);
+            lds_words<4>(wrow, o + 128 + 32 * hf + 16 * h, qh);
+#pragma unroll
+            for (int gi = 0; gi < 4; gi++) {
+              // scale of 16-value group 8 hf + 2 gi + h
+              const uint32_t sw = scw[2 * hf + (gi >> 1)];
+              const int sc = (int)(int8_t)((sw >> (16 * (gi & 1) + 8 * h)) & 0xFFu);
+              const uint32_t sc4 = ((uint32_t)(4 * sc) & 0xFFFFu) * 0x10001u;
+              const uint32_t kb = ((uint32_t)(128 - 128 * sc) & 0xFFFFu) * 0x10001u;
+              i4v bh = {}, bl = {};
+#pragma unroll
+              for (int e = 0; e < 4; e++) {
+                const uint32_t q = ((ql[gi & 1][e] >> (4 * (gi >> 1))) & 0x0F0F0F0Fu) |
+                                   (((qh[e] >> (2 * gi)) & 0x03030303u) << 4);
+                const uint32_t pe = pkmad(q & 0x00FF00FFu, sc4, kb);
+                const uint32_t po = pkmad((q >> 8) & 0x00FF00FFu, sc4, kb);
+                if (which & 1) bh[e] = (int)__builtin_amdgcn_perm(po, pe, 0x07030501u);
+                if (which & 2) bl[e] = (int)(__builtin_amdgcn_perm(po, pe, 0x06020400u) ^ 0x80808080u);
+              }
+              mul(4 * hf + gi, which, bh, bl);
+              if constexpr (MT > 2) __builtin_amdgcn_sched_barrier(0);
+            }
+          }
+        };
+        if constexpr (kWide) {
+          sweep(1);
+          widen();
+          sweep(2);
+        } else {
+          sweep(3);
+        }
+      }
+      // acc += dy (d T - dmin Tm)
+#pragma unroll
+      for (int m = 0; m < MT; m++) {
+        f16v tm = {};
+        if constexpr (!Q6)
+          tm = __builtin_amdgcn_mfma_f32_32x32x16_f16(*(const h8*)&s_bs[cur][32 * m + r32][8 * h], mb, tm, 0, 0, 0);
+#pragma unroll
+        for (int g = 0; g < 4; g++) {
+          const f4v dy4 = *(const f4v*)&s_dy[cur][32 * m + 8 * g + 4 * h];
+#pragma unroll
+          for (int e = 0; e < 4; e++) {
+            const int i = 4 * g + e;
+            const int tt = kWide ? tl[m][i] : (int)(((uint32_t)th[m][i] << (Q6 ? 8 : 3)) + (uint32_t)tl[m][i]);
+            float u;
+            if constexpr (Q6)
+              u = d * (float)tt;
+            else
+              u = __builtin_fmaf(d, (float)tt, -(dmin * tm[i]));
+            acc[m][i] = __builtin_fmaf(dy4[e], u, acc[m][i]);
+          }
+        }
+        // consumed here: the compiler would sink the epilogue past the barrier, holding every tile's tm
+#pragma unroll
+        for (int i = 0; i < 16; i++) asm volatile("" ::"v"(acc[m][i]));
+      }
+      // the next super-block's bytes, in flight since this one's start
+      store_w();
+      store_rows(cur ^ 1);
+      __builtin_amdgcn_s_waitcnt(0);
+      __syncthreads();
+    }
+
+    if (col < N) {
+      float* __restrict__ out = cut ? a.part + pick(a.part_off) + (int64_t)s * M * N + col : dst + col;
+      int64_t ldo = cut ? N : ldd;
+      int hrow = 4 * h;
+      // the rows and their addresses are formed here, not kept live over the K loop
+      asm volatile("" : "+s"(ldo), "+v"(hrow));
+      const bool add = !cut && s > 0;
+#pragma unroll
+      for (int m = 0; m < MT; m++)
+#pragma unroll
+        for (int g = 0; g < 4; g++) {
+          float old[4] = {};
+          if (add) {
+#pragma unroll
+            for (int e = 0; e < 4; e++)
+              if (32 * m + 8 * g + hrow + e < M) old[e] = out[(32 * m + 8 * g + hrow + e) * ldo];
+          }
+#pragma unroll
+          for (int e = 0; e < 4; e++)
+            if (32 * m + 8 * g + hrow + e < M)
+              out[(32 * m + 8 * g + hrow + e) * ldo] = add ? old[e] + acc[m][4 * g + e] : acc[m][4 * g + e];
+        }
+    }
+  }
+}
+
+// dst of the cut weights: the slots added in split order, 4 neighbouring
+// columns a thread where every row of the slots and of dst is 16-byte
+// aligned, else one. blockIdx.y: the weight.
+__global__ __launch_bounds__(256) void gemm_kq_mid_sum_kernel(const MidArgs a) {
+  const int t = (int)blockIdx.y;
+  auto pick = [&](const auto& arr) { return t == 0 ? arr[0] : t == 1 ? arr[1] : t == 2 ? arr[2] : arr[3]; };
+  const int64_t N = pick(a.n), ldd = pick(a.ldd), total = N * a.M;
+  const int S = pick(a.splits);
+  float* __restrict__ dst = pick(a.dst);
+  const float* __restrict__ p = a.part + pick(a.part_off);
+  const uint32_t n32 = (uint32_t)N;  // total < 2^31 (launch_mid)
+  if ((N & 3) == 0 && (ldd & 3) == 0 && ((uintptr_t)dst & 15) == 0) {
+    for (int64_t i = 4 * ((int64_t)blockIdx.x * 256 + threadIdx.x); i < total; i += (int64_t)gridDim.x * 1024) {
+      f4v v = *(const f4v*)(p + i);
+#pragma unroll 4
+      for (int s = 1; s < S; s++) v += *(const f4v*)(p + s * total + i);
+      const uint32_t r = (uint32_t)i / n32;
+      *(f4v*)(dst + r * ldd + ((uint32_t)i - r * n32)) = v;
+    }
+    return;
+  }
+  for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < total; i += (int64_t)gridDim.x * 256) {
+    float v = p[i];
+#pragma unroll 4
+    for (int s = 1; s < S; s++) v += p[s * total + i];
+    const uint32_t r = (uint32_t)i / n32;
+    dst[r * ldd + ((uint32_t)i - r * n32)] = v;
+  }
+}
+
+int tile_cols(int64_t rows) { return rows > 96 ? 256 : 128; }
+
+template <int FMT, int MT, int kNW, bool kWide>
+void launch_kernel(const MidArgs& a, int units, hipStream_t st) {
+  gemm_kq_mid_kernel<FMT, MT, kNW, kWide><<<dim3((unsigned)units), 64 * kNW, 0, st>>>(a);
+}
+
+template <int FMT>
+void launch_fmt(const MidArgs& a, int units, hipStream_t st) {
+  if (a.M <= 32)
+    launch_kernel<FMT, 1, 4, false>(a, units, st);
+  else if (a.M <= 64)
+    launch_kernel<FMT, 2, 4, false>(a, units, st);
+  else if (a.M <= 96)
+    launch_kernel<FMT, 3, 4, false>(a, units, st);
+  else
+    launch_kernel<FMT, 4, 8, true>(a, units, st);
+}
+
+}  // namespace
+
+bool gemm_kq_mid_fits(int type, int64_t n, int64_t k, int64_t rows) {
+  // 32-bit byte offsets inside the kernel
+  const int64_t block = type == T_Q4_K ? 144 : type == T_Q6_K ? 210 : 0;
+  return block != 0 && rows >= kMidMinRows && rows <= kMidMaxRows && k % 256 == 0 &&
+         n * (k / 256) * block + 16 < ((int64_t)1 << 31) && 128 * k < ((int64_t)1 << 31) && n * rows < ((int64_t)1 << 31);
+}
+
+// K ranges of one weight's product, from its own shape (so a weight's bits do
+// not depend on the weights it shares a launch with): as many as bring its
+// workgroups to 256 (128 columns each, two on a CU: gate and up share a
+// launch, and 14336 x 4096 of either gives 224), at least 2 super-blocks a
+// range. Past 96 rows a CU holds one workgroup (256 columns): 128 for the wide
+// weights. Measured at 77 rows, gate + up / q + k + v / down of an 8B layer,
+// slots added: 128 workgroups 54 / 24 / 52 us, 256 45 / 24 / 35, 512 56 / 23 /
+// 36; at 128 rows with 128 / 256 wide workgroups 62 / 76 us for gate + up,
+// 67 / 50 for down.
+int gemm_kq_mid_splits(int64_t n, int64_t k, int64_t rows) {
+  const int64_t bn = tile_cols(rows), tiles = (n + bn - 1) / bn;
+  int64_t s = (bn == 256 && tiles > 32 ? 128 : 256) / tiles;
+  const int64_t most = k / 512;
+  if (s > most) s = most;
+  if (s > 16) s = 16;
+  return s < 1 ? 1 : (int)s;
+}
+
+size_t gemm_kq_mid_slot_bytes(const MvTargets& t, int64_t k, int64_t rows, bool always) {
+  size_t bytes = 0;
+  bool cut = always;
+  for (int i = 0; i < t.count; i++) {
+    const int64_t n = t.row_end[i] - (i ? t.row_end[i - 1] : 0);
+    const int S = gemm_kq_mid_splits(n, k, rows);
+    cut = cut || S > 1;
+    bytes += align_up((size_t)(n * rows) * 4 * S, 256);
+  }
+  return cut ? bytes : 0;
+}
+
+template <int FMT>
+static hipError_t launch_mid(const MvTargets& t, int64_t k, const ActPlanes& p, int64_t rows, void* slots,
+                             size_t slot_bytes, float** parts, hipStream_t st) {
+  if (t.count < 1 || t.count > kMaxTargets) return hipErrorInvalidValue;
+  const size_t need = gemm_kq_mid_slot_bytes(t, k, rows, parts != nullptr);
+  const bool cut = need > 0 && slots != nullptr && slot_bytes >= need;
+  if (parts && !cut) return hipErrorInvalidValue;
+  MidArgs a{};
+  a.yq = p.codes;
+  a.yd = p.d;
+  a.ybs = (const int16_t*)p.sums;
+  a.M = (int)rows;
+  a.nsb = (int)(k / 256);
+  const int64_t bn = tile_cols(rows);
+  int64_t units = 0, floats = 0, most = 0;
+  for (int i = 0; i < kMaxTargets; i++) {
+    const int j = i < t.count ? i : t.count - 1;  // unused entries repeat the last weight, with no units
+    const int64_t n = t.row_end[j] - (j ? t.row_end[j - 1] : 0);
+    a.w[i] = t.w[j];
+    a.dst[i] = t.dst[j];
+    a.ldd[i] = t.ldd[j];
+    a.n[i] = n;
+    a.splits[i] = gemm_kq_mid_splits(n, k, rows);
+    a.part_off[i] = floats;
+    if (i < t.count) {
+      units += (n + bn - 1) / bn * (cut ? a.splits[i] : 1);
+      if (parts) parts[i] = (float*)slots + floats;
+      floats += (int64_t)(align_up((size_t)(n * rows) * 4 * a.splits[i], 256) / 4);
+      most = n * rows > most ? n * rows : most;
+    }
+    a.unit_end[i] = (int)units;
+  }
+  if (units >= ((int64_t)1 << 31)) return hipErrorInvalidValue;
+  a.remap = units % 8 == 0 ? 1 : 0;
+  a.part = cut ? (float*)slots : nullptr;
+  launch_fmt<FMT>(a, (int)units, st);
+  if (cut && !parts) {
+    const int64_t blocks = (most / 4 + 255) / 256;
+    gemm_kq_mid_sum_kernel<<<dim3((unsigned)(blocks < 1 ? 1 : blocks), (unsigned)t.count), 256, 0, st>>>(a);
+  }
+  return hipGetLastError();
+}
+
+hipError_t launch_gemm_q4k_mid(const MvTargets& t, int64_t k, const ActPlanes& p, int64_t rows, void* slots,
+                               size_t slot_bytes, float** parts, hipStream_t st) {
+  QMM_NOTE_LAUNCH();
+  return launch_mid<T_Q4_K>(t, k, p, rows, slots, slot_bytes, parts, st);
+}
+
+hipError_t launch_gemm_q6k(const MvTargets& t, int64_t k, const ActPlanes& p, int64_t rows, void* slots,
+                           size_t slot_bytes, float** parts, hipStream_t st) {
+  QMM_NOTE_LAUNCH();
+  return launch_mid<T_Q6_K>(t, k, p, rows, slots, slot_bytes, parts, st);
+}
+
+}  // namespace qmm

@@ -227,10 +227,17 @@ bool mmq_allows(int64_t rows) {
 
 bool aligned16(const void* p) { return ((uintptr_t)p & 15) == 0; }
 
+// Q4_K and Q6_K at 17-128 rows (gemm_kq_mid.hip): all activation rows in one
+// workgroup tile, the weight cut along K.
+bool mid_takes(int type, const void* w, const void* xq, int64_t n, int64_t k, int64_t rows) {
+  return mmq_allows(rows) && aligned16(w) && aligned16(xq) && qmm::gemm_kq_mid_fits(type, n, k, rows);
+}
+
 // The few-row matrix-core kernels (Q4_K, Q6_K): up to
-// gemm_q4k_skinny_max_rows() rows past the few-rows line.
+// gemm_q4k_skinny_max_rows() rows past the few-rows line that mid_takes leaves.
 bool skinny_takes(int type, const void* w, const void* xq, int64_t n, int64_t k, int64_t rows, hipStream_t st) {
   if (!mmq_allows(rows) || rows > qmm::gemm_q4k_skinny_max_rows() || !aligned16(w) || !aligned16(xq)) return false;
+  if (mid_takes(type, w, xq, n, k, rows)) return false;
   int64_t wbytes;
   if (type == qmm::T_Q4_K && qmm::gemm_q4k_skinny_fits(k, rows))
     wbytes = n * (k / 256) * 144;
@@ -262,13 +269,20 @@ bool gemm_takes(int type, const void* w, const void* xq, int64_t n, int64_t k, i
   return few_rows_take(type, rows, n * (k / 32) * type_size(type), st);
 }
 
-// Whether a product goes to a matrix-core kernel rather than the decode kernels.
-bool matrix_takes(int type, const void* w, const void* xq, int64_t n, int64_t k, int64_t rows, hipStream_t st) {
-  return gemm_takes(type, w, xq, n, k, rows, st) || skinny_takes(type, w, xq, n, k, rows, st);
+hipError_t launch_mid(int type, const qmm::MvTargets& t, int64_t k, const qmm::ActPlanes& p, int64_t rows, void* slots,
+                      size_t slot_bytes, float** parts, hipStream_t st) {
+  return type == qmm::T_Q6_K ? qmm::launch_gemm_q6k(t, k, p, rows, slots, slot_bytes, parts, st)
+                             : qmm::launch_gemm_q4k_mid(t, k, p, rows, slots, slot_bytes, parts, st);
 }
 
-// Q4_K: from 129 rows the single-pass GEMM (256-row tiles); 33-128 rows keep
-// the exact two-pass kernel, whose 128-row tiles waste less on short batches.
+// Whether a product goes to a matrix-core kernel rather than the decode kernels.
+bool matrix_takes(int type, const void* w, const void* xq, int64_t n, int64_t k, int64_t rows, hipStream_t st) {
+  return mid_takes(type, w, xq, n, k, rows) || gemm_takes(type, w, xq, n, k, rows, st) ||
+         skinny_takes(type, w, xq, n, k, rows, st);
+}
+
+// Past mid_takes' rows. Q4_K: the single-pass GEMM (256-row tiles); rows
+// shorter than its k keep the exact two-pass kernel.
 hipError_t launch_gemm(int type, const void* w, int64_t n, int64_t k, const qmm::ActPlanes& p, int64_t rows,
                        float* dst, int64_t ldd, hipStream_t st) {
   if (qmm::exact_forms()) {
@@ -311,6 +325,21 @@ qmm::MvTargets one_target(const void* w, int64_t n, float* dst, int64_t ldd) {
   t.ldd[0] = ldd;
   t.row_end[0] = n;
   t.count = 1;
+  return t;
+}
+
+// Weights i0 .. of a shared product, at most kMaxTargets.
+qmm::MvTargets targets_of(const void* const* w, const int64_t* n, float* const* dst, const int64_t* ldd, int i0,
+                          int count) {
+  qmm::MvTargets t{};
+  int64_t end = 0;
+  for (int i = i0; i < count && t.count < qmm::kMaxTargets; i++) {
+    t.w[t.count] = w[i];
+    t.dst[t.count] = dst[i];
+    t.ldd[t.count] = ldd[i];
+    end += n[i];
+    t.row_end[t.count++] = end;
+  }
   return t;
 }
 
@@ -547,6 +576,12 @@ int qmm_matvec(int type, const void* w, const void* xq, float* dst, int64_t ldd,
 // kernels a chunk of at most matvec_max_rows() rows at a time.
 int launch_product(int type, const void* w, int64_t n, int64_t k, const void* xq, const qmm::ActPlanes& p,
                    int layout, int64_t rows, float* dst, int64_t ldd, hipStream_t st) {
+  if (mid_takes(type, w, xq, n, k, rows)) {
+    if (launch_mid(type, one_target(w, n, dst, ldd), k, p, rows, nullptr, 0, nullptr, st) != hipSuccess)
+      return QMM_DEVICE_ERROR;
+    g_gemm_launches.fetch_add(1, std::memory_order_relaxed);
+    return QMM_OK;
+  }
   if (gemm_takes(type, w, xq, n, k, rows, st)) {
     if (launch_gemm(type, w, n, k, p, rows, dst, ldd, st) != hipSuccess) return QMM_DEVICE_ERROR;
     g_gemm_launches.fetch_add(1, std::memory_order_relaxed);
@@ -595,7 +630,9 @@ int qmm_forward(int type, const void* w, const float* x, int64_t x_stride, float
   // a single-pass GEMM that leaves CUs idle is cut along K when the
   // workspace also holds its split slots (need reports them; with only the
   // activation's bytes it runs uncut)
-  const size_t split = sp_takes(type, w, workspace, n, k, rows, st)
+  const bool mid = mid_takes(type, w, workspace, n, k, rows);
+  const size_t split = mid ? qmm::gemm_kq_mid_slot_bytes(one_target(w, n, dst, ldd), k, rows, false)
+                       : sp_takes(type, w, workspace, n, k, rows, st)
                            ? qmm::gemm_q4k_sp_split_bytes(one_target(w, n, dst, ldd), k, rows, (int)cu_count())
                            : 0;
   *need = split ? qmm::align_up(bytes, 256) + split : bytes;
@@ -617,9 +654,16 @@ int qmm_forward(int type, const void* w, const float* x, int64_t x_stride, float
   if (qmm::launch_act_quantize(layout, x, x_stride, k, rows, workspace, q8k_scale(), st) != hipSuccess)
     return QMM_DEVICE_ERROR;
   const qmm::ActPlanes p = qmm::act_planes(layout, workspace, k, rows);
+  if (mid && split && workspace_bytes >= *need) {
+    if (launch_mid(type, one_target(w, n, dst, ldd), k, p, rows, (char*)workspace + qmm::align_up(bytes, 256), split,
+                   nullptr, st) != hipSuccess)
+      return QMM_DEVICE_ERROR;
+    g_gemm_launches.fetch_add(1, std::memory_order_relaxed);
+    return QMM_OK;
+  }
   // Q6_K takes the single-pass GEMM only cut as planned (uncut, a narrow
   // product runs faster on the exact kernel)
-  if (sp_takes(type, w, workspace, n, k, rows, st) &&
+  if (!mid && sp_takes(type, w, workspace, n, k, rows, st) &&
       (type == qmm::T_Q4_K || split == 0 || workspace_bytes >= *need)) {
     const size_t off = qmm::align_up(bytes, 256);
     void* sws = workspace_bytes > off ? (char*)workspace + off : nullptr;
@@ -641,10 +685,17 @@ int qmm_forward_shared(int type, int count, const void* const* w, const int64_t*
   const int layout = qmm_act_layout(type, rows);
   const size_t bytes = qmm::act_bytes(layout, k, rows);
   const hipStream_t st = (hipStream_t)stream;
-  // the single-pass GEMM's products go kMaxTargets to a launch; their split
-  // slots follow the activation (one launch's worth, reused launch after launch)
+  // the 17-128 row kernel's and the single-pass GEMM's products go
+  // kMaxTargets to a launch; their split slots follow the activation (one
+  // launch's worth, reused launch after launch)
   size_t split = 0;
-  {
+  bool mid = true;  // the rows and type decide, and the weights' sizes and alignment
+  for (int i = 0; i < count; i++) mid = mid && mid_takes(type, w[i], workspace, n[i], k, rows);
+  for (int i0 = 0; mid && i0 < count; i0 += qmm::kMaxTargets) {
+    const size_t b = qmm::gemm_kq_mid_slot_bytes(targets_of(w, n, dst, ldd, i0, count), k, rows, false);
+    split = b > split ? b : split;
+  }
+  if (!mid) {
     qmm::MvTargets g{};
     int64_t end = 0;
     for (int i = 0; i <= count; i++) {
@@ -695,6 +746,16 @@ int qmm_forward_shared(int type, int count, const void* const* w, const int64_t*
   if (qmm::launch_act_quantize(layout, x, x_stride, k, rows, workspace, q8k_scale(), st) != hipSuccess)
     return QMM_DEVICE_ERROR;
   const qmm::ActPlanes p = qmm::act_planes(layout, workspace, k, rows);
+  if (mid) {
+    void* slots = split && workspace_bytes >= *need ? (char*)workspace + qmm::align_up(bytes, 256) : nullptr;
+    for (int i0 = 0; i0 < count; i0 += qmm::kMaxTargets) {
+      if (launch_mid(type, targets_of(w, n, dst, ldd, i0, count), k, p, rows, slots, slots ? split : 0, nullptr, st) !=
+          hipSuccess)
+        return QMM_DEVICE_ERROR;
+      g_gemm_launches.fetch_add(1, std::memory_order_relaxed);
+    }
+    return QMM_OK;
+  }
   // the weights the skinny kernel takes share its launches (kMaxTargets
   // each), and so do those the single-pass GEMM takes
   qmm::MvTargets grp{}, spg{};
@@ -759,7 +820,15 @@ int qmm_forward_glu(int type, int act, const void* w_gate, const void* w_up, con
   const size_t abytes = qmm::act_bytes(layout, k, rows);
   const size_t obytes = qmm::align_up((size_t)(rows * n) * 4, 256);
   const size_t bytes = abytes + 2 * obytes;
-  *need = bytes;
+  // at 17-128 rows the GLU adds the products' K-split slots itself, when the
+  // workspace holds them
+  const bool mid = mid_takes(type, w_gate, workspace, n, k, rows) && mid_takes(type, w_up, workspace, n, k, rows);
+  const void* w[2] = {w_gate, w_up};
+  const int64_t ns[2] = {n, n};
+  float* none[2] = {nullptr, nullptr};
+  const size_t aoff = qmm::align_up(abytes, 256);
+  const size_t slots = mid ? qmm::gemm_kq_mid_slot_bytes(targets_of(w, ns, none, ns, 0, 2), k, rows, true) : 0;
+  *need = aoff + slots > bytes ? aoff + slots : bytes;
   if (!launch) return QMM_OK;
   if (g_fail_next.exchange(false)) return QMM_NO_ROOM;
   if (!w_gate || !w_up || !x || !dst) return QMM_UNSUPPORTED;
@@ -775,10 +844,20 @@ int qmm_forward_glu(int type, int act, const void* w_gate, const void* w_up, con
     return QMM_OK;
   }
   if (workspace_bytes < bytes || workspace == nullptr) return QMM_WORKSPACE_TOO_SMALL;
+  if (mid && workspace_bytes >= aoff + slots && !g_force_dmmv.load(std::memory_order_relaxed)) {
+    if (qmm::launch_act_quantize(layout, x, x_stride, k, rows, workspace, q8k_scale(), st) != hipSuccess)
+      return QMM_DEVICE_ERROR;
+    const qmm::ActPlanes p = qmm::act_planes(layout, workspace, k, rows);
+    float* parts[2];
+    if (launch_mid(type, targets_of(w, ns, none, ns, 0, 2), k, p, rows, (char*)workspace + aoff, slots, parts, st) !=
+        hipSuccess)
+      return QMM_DEVICE_ERROR;
+    g_gemm_launches.fetch_add(1, std::memory_order_relaxed);
+    return status_of(qmm::launch_glu(act, parts[0], parts[1], qmm::gemm_kq_mid_splits(n, k, rows), dst, ldd, n, rows,
+                                     st));
+  }
   float* gbuf = (float*)((char*)workspace + abytes);
   float* ubuf = (float*)((char*)gbuf + obytes);
-  const void* w[2] = {w_gate, w_up};
-  const int64_t ns[2] = {n, n};
   float* outs[2] = {gbuf, ubuf};
   size_t need2 = 0;
   const int r = qmm_forward_shared(type, 2, w, ns, outs, ns, x, x_stride, workspace, abytes, &need2, k, rows, 1,

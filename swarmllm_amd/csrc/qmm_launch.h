@@ -184,6 +184,10 @@ hipError_t launch_mv_q4k_glu(int act, const void* wg, const void* wu, int64_t n,
                              int cus, hipStream_t st);
 hipError_t launch_glu(int act, const float* gate, int64_t ldg, const float* up, int64_t ldu, float* out, int64_t ldo,
                       int64_t n, int64_t rows, hipStream_t st);
+// The same over gate and up products left in `splits` slots of rows x n
+// values each, added in slot order first.
+hipError_t launch_glu(int act, const float* gate, const float* up, int splits, float* out, int64_t ldo, int64_t n,
+                      int64_t rows, hipStream_t st);
 
 // The Q8_0 hidden-state wire codec (wire.hip): bytes of n values (-1 when
 // they would not fit an int64), encode, decode.
@@ -215,6 +219,23 @@ hipError_t launch_gemm_q6k_sp(const void* w, int64_t n, int64_t k, const ActPlan
                               int64_t ldd, hipStream_t s);
 hipError_t launch_gemm_q6k_sp_targets(const MvTargets& t, int64_t k, const ActPlanes& p, int64_t rows, void* split_ws,
                                       size_t split_bytes, int cus, hipStream_t st);
+
+// Q4_K and Q6_K products of 17 to 128 rows (gemm_kq_mid.hip): exact int32
+// super-block sums, each weight cut along K into gemm_kq_mid_splits ranges
+// (from its own shape). Bytes of the slots of a launch over `t` (0: no weight
+// is cut, unless `always`). The launch, with slots of that size: the partial
+// products to the slots and a second launch adding them into dst in split
+// order, or with `parts` (slots of the `always` size) the slots left to the
+// caller ([split][rows][n] at parts[i]); without them a workgroup adds a
+// tile's splits into dst one after another: the same bits.
+constexpr int kMidMinRows = 17, kMidMaxRows = 128;
+bool gemm_kq_mid_fits(int type, int64_t n, int64_t k, int64_t rows);
+int gemm_kq_mid_splits(int64_t n, int64_t k, int64_t rows);
+size_t gemm_kq_mid_slot_bytes(const MvTargets& t, int64_t k, int64_t rows, bool always);
+hipError_t launch_gemm_q4k_mid(const MvTargets& t, int64_t k, const ActPlanes& p, int64_t rows, void* slots,
+                               size_t slot_bytes, float** parts, hipStream_t st);
+hipError_t launch_gemm_q6k(const MvTargets& t, int64_t k, const ActPlanes& p, int64_t rows, void* slots,
+                           size_t slot_bytes, float** parts, hipStream_t st);
 
 int gemm_q4k_min_rows();
 // The GEMM indexes with 32-bit byte offsets: the weight below 2 GiB and

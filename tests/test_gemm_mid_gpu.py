@@ -1,0 +1,128 @@
+"""Q4_K and Q6_K products of 17-128 rows (gemm_kq_mid.hip) against the CPU
+oracle: at the edges of its row tiles (32, 64, 96, 128), of its column tiles
+(128, and 256 past 96 rows) and of its K cut, and with the largest codes and
+scales a block can hold.
+
+Bound: the super-block sums are exact integers and the min sums exact f32, so
+a result differs from the oracle's by f32 roundings only: per super-block
+three (2^-24 each) of terms bounded by d dy sum |p y| + dmin dy sum |m S| and
+one per addition, so at most (nsb + 4) 2^-24 of the sum of the terms'
+magnitudes, which for these weights is below 3 ||w|| ||x||: 1.1e-5 at 56
+super-blocks; 1e-5 is held (1e-7 measured)."""
+import ctypes
+import zlib
+
+import numpy as np
+import pytest
+import torch
+
+from helpers import normalised_error, special_rows, weights
+from oracle import qref
+from swarmllm_amd import GgmlDType, QMatMul, QTensor, _lib
+from swarmllm_amd._lib import lib
+from swarmllm_amd.qtensor import quantize_act
+
+pytestmark = pytest.mark.gpu
+
+BOUND = 1e-5
+KERNEL = {qref.Q4_K: "launch_gemm_q4k_mid(", qref.Q6_K: "launch_gemm_q6k("}
+
+SHAPES = [  # (n, k, rows)
+    (1, 256, 17), (127, 512, 32), (129, 1024, 33), (128, 768, 64), (300, 4096, 65), (2048, 2048, 96),
+    (255, 512, 97), (257, 2560, 128), (1024, 14336, 50), (9000, 512, 100),
+]
+
+
+def stream():
+    return torch.cuda.current_stream().cuda_stream
+
+
+def forward(t, qt, x, n, k, rows, ws_bytes=None):
+    L = lib()
+    out = torch.full((rows, n), float("nan"), dtype=torch.float32, device="cuda")
+    need = ctypes.c_size_t(0)
+    assert L.qmm_forward(t, None, None, k, None, n, None, 0, ctypes.byref(need), k, n, rows, 0, 0) == 0
+    ws = torch.empty(ws_bytes or need.value, dtype=torch.uint8, device="cuda")
+    assert L.qmm_forward(t, qt.data_.data_ptr(), x.data_ptr(), k, out.data_ptr(), n, ws.data_ptr(), ws.numel(),
+                         ctypes.byref(need), k, n, rows, 1, stream()) == 0
+    return out, need.value
+
+
+@pytest.mark.parametrize("t", [qref.Q4_K, qref.Q6_K], ids=["q4k", "q6k"])
+@pytest.mark.parametrize("n,k,rows", SHAPES)
+def test_against_the_oracle_and_the_same_bits_whatever_the_workspace(t, n, k, rows):
+    rng = np.random.default_rng(zlib.crc32(f"mid-{t}-{n}-{k}-{rows}".encode()))
+    wq = qref.from_float(t, weights(rng, n, k))
+    qt = QTensor.from_data(wq.tobytes(), (n, k), GgmlDType(t))
+    x = rng.standard_normal((rows, k)).astype(np.float32)
+    xt = torch.from_numpy(x).cuda()
+    print(f"t={t} n={n} k={k} rows={rows}", flush=True)
+    y, need = forward(t, qt, xt, n, k, rows)
+    assert KERNEL[t] in lib().qmm_last_kernel().decode()
+    want = qref.matmul(t, x, wq, n)
+    wdeq = qref.to_float(t, wq, n * k).reshape(n, k)
+    err = normalised_error(y.cpu().numpy(), want, wdeq, x)
+    assert err <= BOUND, err
+    # no room for the split slots: a workgroup adds a tile's splits in turn
+    act = lib().qmm_act_bytes(_lib.ACT_Q8K, k, rows)
+    assert torch.equal(forward(t, qt, xt, n, k, rows, act)[0], y)
+    assert torch.equal(forward(t, qt, xt, n, k, rows, need - 1)[0], y) if need > act else True
+    xq = quantize_act(xt, _lib.ACT_Q8K)
+    out = torch.empty_like(y)
+    assert lib().qmm_matmul(t, qt.data_.data_ptr(), xq.data_ptr(), out.data_ptr(), n, k, n, rows, stream()) == 0
+    assert torch.equal(out, y)
+
+
+@pytest.mark.parametrize("rows", [20, 77, 128])
+def test_shared_products_keep_each_weights_bits(rows):
+    """Five weights (two launches) of which some are cut and some are not."""
+    k = 4096
+    mats = []
+    for i, n in enumerate((2048, 256, 33, 12000, 130)):
+        rng = np.random.default_rng(400 + i)
+        wq = qref.from_float(qref.Q4_K, weights(rng, n, k))
+        mats.append(QMatMul(QTensor.from_data(wq.tobytes(), (n, k), GgmlDType.Q4K)))
+    x = torch.from_numpy(np.random.default_rng(9).standard_normal((rows, k)).astype(np.float32)).cuda()
+    for m, y in zip(mats, QMatMul.forward_shared(x, mats)):
+        assert torch.equal(y, m.forward(x))
+
+
+@pytest.mark.parametrize("rows", [30, 128])
+def test_padded_output_rows_stay_untouched(rows):
+    """ldd > n and an n that is no multiple of 4: nothing past a row's n."""
+    t, n, k, ldd = qref.Q4_K, 1023, 4096, 1030
+    rng = np.random.default_rng(17)
+    wq = qref.from_float(t, weights(rng, n, k))
+    qt = QTensor.from_data(wq.tobytes(), (n, k), GgmlDType(t))
+    x = torch.from_numpy(rng.standard_normal((rows, k)).astype(np.float32)).cuda()
+    y, need = forward(t, qt, x, n, k, rows)
+    out = torch.full((rows, ldd), float("nan"), dtype=torch.float32, device="cuda")
+    ws = torch.empty(need, dtype=torch.uint8, device="cuda")
+    nd = ctypes.c_size_t(0)
+    assert lib().qmm_forward(t, qt.data_.data_ptr(), x.data_ptr(), k, out.data_ptr(), ldd, ws.data_ptr(), ws.numel(),
+                             ctypes.byref(nd), k, n, rows, 1, stream()) == 0
+    assert torch.equal(out[:, :n], y) and bool(torch.isnan(out[:, n:]).all())
+
+
+def test_q4k_largest_codes_scales_and_mins():
+    """Blocks of q = 15 with scales and mins of 63 (sc q = 945, the largest
+    operand products 105) against rows of one sign (|T| near 2^24.9, |Tm| near
+    2^21), the quantizer's edge rows, and rows scaled by 1e-30 and 1e30."""
+    n, k = 64, 2048
+    rng = np.random.default_rng(77)
+    wq = qref.from_float(qref.Q4_K, weights(rng, n, k)).view(np.uint8).reshape(n * k // 256, 144).copy()
+    # get_scale_min_k4's packing of 63 everywhere is all ones
+    wq[::2, 4:16] = 0xFF
+    wq[::2, 16:] = 0xFF
+    wq = wq.reshape(-1)
+    qt = QTensor.from_data(wq.tobytes(), (n, k), GgmlDType.Q4K)
+    sp = special_rows(k)
+    x = np.concatenate([sp, np.full((3, k), 1.0, np.float32), rng.standard_normal((20, k)).astype(np.float32)])
+    x[len(sp) + 1] *= -1.0
+    x[-1] *= np.float32(1e-30)
+    x[-2] *= np.float32(1e30)
+    y = QMatMul(qt).forward(torch.from_numpy(x).cuda()).cpu().numpy()
+    assert np.all(y[0] == 0.0)
+    want = qref.matmul(qref.Q4_K, x, wq, n)
+    wdeq = qref.to_float(qref.Q4_K, wq, n * k).reshape(n, k)
+    assert normalised_error(y, want, wdeq, x) <= BOUND
