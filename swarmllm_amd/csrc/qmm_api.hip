@@ -281,6 +281,16 @@ bool matrix_takes(int type, const void* w, const void* xq, int64_t n, int64_t k,
          skinny_takes(type, w, xq, n, k, rows, st);
 }
 
+qmm::MvTargets one_target(const void* w, int64_t n, float* dst, int64_t ldd) {
+  qmm::MvTargets t{};
+  t.w[0] = w;
+  t.dst[0] = dst;
+  t.ldd[0] = ldd;
+  t.row_end[0] = n;
+  t.count = 1;
+  return t;
+}
+
 // Past mid_takes' rows. Q4_K: the single-pass GEMM (256-row tiles); rows
 // shorter than its k keep the exact two-pass kernel.
 hipError_t launch_gemm(int type, const void* w, int64_t n, int64_t k, const qmm::ActPlanes& p, int64_t rows,
@@ -298,7 +308,7 @@ hipError_t launch_gemm(int type, const void* w, int64_t n, int64_t k, const qmm:
       return qmm::launch_gemm_q6k_sp(w, n, k, p, rows, dst, ldd, st);
     return qmm::launch_gemm_q6k(w, n, k, p, rows, dst, ldd, st);
   }
-  if (type != qmm::T_Q4_K) return qmm::launch_gemm_b32(type, w, n, k, p, rows, dst, ldd, st);
+  if (type != qmm::T_Q4_K) return qmm::launch_gemm_b32(type, one_target(w, n, dst, ldd), k, p, rows, st);
   if (rows >= qmm::gemm_q4k_sp_min_rows() && qmm::gemm_q4k_sp_fits(n, k, rows))
     return qmm::launch_gemm_q4k_sp(w, n, k, p, rows, dst, ldd, st);
   return qmm::launch_gemm_q4k(w, n, k, p, rows, dst, ldd, st);
@@ -316,16 +326,6 @@ hipError_t launch_sp(int type, const qmm::MvTargets& t, int64_t k, const qmm::Ac
                      size_t ws_bytes, hipStream_t st) {
   return type == qmm::T_Q6_K ? qmm::launch_gemm_q6k_sp_targets(t, k, p, rows, ws, ws_bytes, (int)cu_count(), st)
                              : qmm::launch_gemm_q4k_sp_targets(t, k, p, rows, ws, ws_bytes, (int)cu_count(), st);
-}
-
-qmm::MvTargets one_target(const void* w, int64_t n, float* dst, int64_t ldd) {
-  qmm::MvTargets t{};
-  t.w[0] = w;
-  t.dst[0] = dst;
-  t.ldd[0] = ldd;
-  t.row_end[0] = n;
-  t.count = 1;
-  return t;
 }
 
 // Weights i0 .. of a shared product, at most kMaxTargets.
@@ -755,6 +755,18 @@ int qmm_forward_shared(int type, int count, const void* const* w, const int64_t*
       g_gemm_launches.fetch_add(1, std::memory_order_relaxed);
     }
     return QMM_OK;
+  }
+  if (!is_kquant(type)) {
+    bool gemm = true;
+    for (int i = 0; i < count; i++) gemm = gemm && gemm_takes(type, w[i], workspace, n[i], k, rows, st);
+    if (gemm) {
+      for (int i0 = 0; i0 < count; i0 += qmm::kMaxTargets) {
+        if (qmm::launch_gemm_b32(type, targets_of(w, n, dst, ldd, i0, count), k, p, rows, st) != hipSuccess)
+          return QMM_DEVICE_ERROR;
+        g_gemm_launches.fetch_add(1, std::memory_order_relaxed);
+      }
+      return QMM_OK;
+    }
   }
   // the weights the skinny kernel takes share its launches (kMaxTargets
   // each), and so do those the single-pass GEMM takes
