@@ -465,9 +465,20 @@ void launch_fmt(const MidArgs& a, int units, hipStream_t st) {
 
 }  // namespace
 
+// The products this kernel takes. Up to 32 rows the few-row kernels, which
+// need no second launch, keep the smaller weights (this kernel against them at
+// 17 / 32 rows, one launch each: Q4_K 4096 x 4096 14.5 / 15.5 us against 10.7 /
+// 12.3, 8192 x 8192 23.6 / 24.5 against 22.7 / 27.9, 4096 x 14336 22.6 / 23.8
+// against 21.8 / 24.8, 14336 x 4096 22.5 / 23.5 against 23.9 / 29.2, 8192 x
+// 28672 57 / 61 against 64 / 79; Q6_K alike): it takes those of 14336 x 4096
+// values, below 24 rows only the wide ones and those over twice that.
 bool gemm_kq_mid_fits(int type, int64_t n, int64_t k, int64_t rows) {
-  // 32-bit byte offsets inside the kernel
   const int64_t block = type == T_Q4_K ? 144 : type == T_Q6_K ? 210 : 0;
+  if (rows <= 32) {
+    constexpr int64_t kLarge = (int64_t)14336 * 4096;
+    if (n * k < kLarge || (rows < 24 && n < 14336 && n * k < 2 * kLarge)) return false;
+  }
+  // 32-bit byte offsets inside the kernel
   return block != 0 && rows >= kMidMinRows && rows <= kMidMaxRows && k % 256 == 0 &&
          n * (k / 256) * block + 16 < ((int64_t)1 << 31) && 128 * k < ((int64_t)1 << 31) && n * rows < ((int64_t)1 << 31);
 }

@@ -28,7 +28,7 @@ BOUND = 1e-5
 KERNEL = {qref.Q4_K: "launch_gemm_q4k_mid(", qref.Q6_K: "launch_gemm_q6k("}
 
 SHAPES = [  # (n, k, rows)
-    (1, 256, 17), (127, 512, 32), (129, 1024, 33), (128, 768, 64), (300, 4096, 65), (2048, 2048, 96),
+    (129, 1024, 33), (1, 256, 40), (128, 768, 64), (300, 4096, 65), (2048, 2048, 96),
     (255, 512, 97), (257, 2560, 128), (1024, 14336, 50), (9000, 512, 100),
 ]
 
@@ -73,7 +73,30 @@ def test_against_the_oracle_and_the_same_bits_whatever_the_workspace(t, n, k, ro
     assert torch.equal(out, y)
 
 
-@pytest.mark.parametrize("rows", [20, 77, 128])
+LARGE = [  # up to 32 rows: the sizes the few-row kernels leave (n, k, rows, taken)
+    (14336, 4096, 17, True), (14335, 4096, 32, False), (4096, 14336, 24, True), (4096, 14336, 23, False),
+    (14340, 4096, 31, True), (8192, 14336, 17, True),
+]
+
+
+@pytest.mark.parametrize("t", [qref.Q4_K, qref.Q6_K], ids=["q4k", "q6k"])
+@pytest.mark.parametrize("n,k,rows,taken", LARGE)
+def test_large_weights_up_to_32_rows(t, n, k, rows, taken):
+    from swarmllm_amd import fill_normal
+
+    qt = QTensor.quantize(fill_normal(n * k, seed=n + k, std=0.02).reshape(n, k), GgmlDType(t))
+    xt = fill_normal(rows * k, seed=rows).reshape(rows, k)
+    print(f"t={t} n={n} k={k} rows={rows}", flush=True)
+    y, need = forward(t, qt, xt, n, k, rows)
+    assert (KERNEL[t] in lib().qmm_last_kernel().decode()) == taken
+    x, wq = xt.cpu().numpy(), qt.data_.cpu().numpy()
+    err = normalised_error(y.cpu().numpy(), qref.matmul(t, x, wq, n), qt.dequantize().cpu().numpy(), x)
+    assert err <= (BOUND if taken or t == qref.Q4_K else 1e-3), err  # few-row Q6_K: its single-product form
+    act = lib().qmm_act_bytes(_lib.ACT_Q8K, k, rows)
+    assert torch.equal(forward(t, qt, xt, n, k, rows, act)[0], y)
+
+
+@pytest.mark.parametrize("rows", [33, 77, 128])
 def test_shared_products_keep_each_weights_bits(rows):
     """Five weights (two launches) of which some are cut and some are not."""
     k = 4096
@@ -87,7 +110,7 @@ def test_shared_products_keep_each_weights_bits(rows):
         assert torch.equal(y, m.forward(x))
 
 
-@pytest.mark.parametrize("rows", [30, 128])
+@pytest.mark.parametrize("rows", [40, 128])
 def test_padded_output_rows_stay_untouched(rows):
     """ldd > n and an n that is no multiple of 4: nothing past a row's n."""
     t, n, k, ldd = qref.Q4_K, 1023, 4096, 1030
@@ -117,7 +140,7 @@ def test_q4k_largest_codes_scales_and_mins():
     wq = wq.reshape(-1)
     qt = QTensor.from_data(wq.tobytes(), (n, k), GgmlDType.Q4K)
     sp = special_rows(k)
-    x = np.concatenate([sp, np.full((3, k), 1.0, np.float32), rng.standard_normal((20, k)).astype(np.float32)])
+    x = np.concatenate([sp, np.full((3, k), 1.0, np.float32), rng.standard_normal((30, k)).astype(np.float32)])
     x[len(sp) + 1] *= -1.0
     x[-1] *= np.float32(1e-30)
     x[-2] *= np.float32(1e30)
