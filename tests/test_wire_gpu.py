@@ -56,3 +56,26 @@ def test_wire_rejects_a_wrong_length_and_takes_empty_input():
     assert st == QMM_UNSUPPORTED
     assert quant.quantize_q8_0(torch.empty(0, device="cuda")).numel() == 0
     assert quant.dequantize_q8_0(torch.empty(0, dtype=torch.uint8, device="cuda"), 0).numel() == 0
+
+
+@pytest.mark.parametrize("n", [7, 2047, 2048, 2049, 2056, 5 * 2048 + 40])
+@pytest.mark.parametrize("xo,bo", [(0, 0), (1, 0), (0, 1), (3, 5), (4, 16)])
+def test_wire_at_any_alignment_and_workgroup_edge(n, xo, bo):
+    """Values and bytes at any offset from a 16-byte boundary (the vector
+    accesses step aside) and lengths around a workgroup's 2048 values; nothing
+    is written past the last byte or value."""
+    x = inputs(n, n + xo)
+    xb = torch.zeros(n + xo, device="cuda")
+    xb[xo:] = torch.from_numpy(x).cuda()
+    want = qref.wire_encode(x)
+    nb = want.size
+    out = torch.full((bo + nb + 64,), 0xA5, dtype=torch.uint8, device="cuda")
+    st = torch.cuda.current_stream().cuda_stream
+    assert lib().qmm_wire_encode(xb.data_ptr() + 4 * xo, n, out.data_ptr() + bo, st) == 0
+    got = out.cpu().numpy()
+    assert np.array_equal(got[bo:bo + nb], want) and np.all(got[bo + nb:] == 0xA5) and np.all(got[:bo] == 0xA5)
+    y = torch.full((xo + n + 16,), -7.0, device="cuda")
+    assert lib().qmm_wire_decode(out.data_ptr() + bo, nb, n, y.data_ptr() + 4 * xo, st) == 0
+    y = y.cpu().numpy()
+    assert np.array_equal(y[xo:xo + n].view(np.uint32), qref.wire_decode(want, n).view(np.uint32))
+    assert np.all(y[xo + n:] == -7.0) and np.all(y[:xo] == -7.0)
