@@ -240,10 +240,11 @@ enum qmm_glu_act_id {
  * activation, and the gated activation between them, written once. For Q4_K
  * at 1-2 rows and k <= 8192 with a 16-byte aligned activation this is ONE
  * launch (each wave computes gate row j and up row j and writes the product;
- * the activation quantized in LDS); otherwise the two products run as
- * qmm_forward_shared into the workspace, followed by the elementwise GLU.
- * Either way the results equal qmm_forward_shared followed by qmm_glu bit for
- * bit. Plan (launch == 0) and launch as qmm_forward. Replaces the
+ * the activation quantized in LDS), and past 128 rows one launch of the
+ * single-pass GEMM, neither weight cut along K; otherwise the two products run
+ * as qmm_forward_shared into the workspace, followed by the elementwise GLU.
+ * The results equal the two products (uncut past 128 rows) followed by
+ * qmm_glu bit for bit. Plan (launch == 0) and launch as qmm_forward. Replaces the
  * reference's forward_shared of ffn_up and ffn_gate followed by silu_mul /
  * swiglu_oai_mul / the GELU product (src/inference/layers/mod.rs:583-632). */
 int qmm_forward_glu(int type, int act, const void *w_gate, const void *w_up, const float *x, int64_t x_stride,

@@ -45,6 +45,7 @@
 //     by the threads during its first half and read by its epilogue.
 // Rows past M and weight rows past N are read as the last row (valid
 // memory); their outputs are never stored.
+#include "glu_act.h"
 #include "lds_copy.h"
 #include "qmm_device.h"
 #include "qmm_launch.h"
@@ -197,10 +198,17 @@ __device__ __forceinline__ void build_q6(uint32_t wr, int half, uint32_t w0, uin
   }
 }
 
-template <int FMT>
+// GLU >= 0: the workgroup's tile is 64 rows of the gate weight (targets 0) and
+// the same 64 of the up weight (target 1), a wave's two column tiles 32 of
+// each, and dst (target 0's) takes act(gate) * up: the same sums as the two
+// products', without writing and reading them (Q4_K, uncut). An 8B layer's gate
+// + up + SiLU at 512 rows 132 -> 119 us, at 2000 475 -> 422.
+template <int FMT, int GLU>
 __global__ __launch_bounds__(kThreads, 1) void gemm_kq_sp_kernel(const SpArgs a) {
   using F = SpFmt<FMT>;
   constexpr bool Q6 = F::kQ6;
+  constexpr int kCols = GLU < 0 ? kBN : kBN / 2;  // columns of dst a workgroup writes
+  static_assert(GLU < 0 || !Q6, "the gated form is Q4_K's");
   // Each half of each double buffer is its own object and the stage loop is
   // unrolled over two super-blocks, so every access names its buffer
   // statically (the compiler can tell reads of one half from writes of the other).
@@ -247,7 +255,7 @@ __global__ __launch_bounds__(kThreads, 1) void gemm_kq_sp_kernel(const SpArgs a)
   // product, 512 x 14336 cut in 4: 1.8 MB an XCD, which its L2 holds; with
   // the splits fastest every XCD read the whole 7.3 MB activation)
   const int64_t N = pick(a.n);
-  const int ctiles = (int)((N + kBN - 1) / kBN);
+  const int ctiles = (int)((N + kCols - 1) / kCols);
   const int mt = loc % mtiles, rest = loc / mtiles;
   const int ct = rest % ctiles, split = (rest / ctiles) * P;
   const uint8_t* __restrict__ W = (const uint8_t*)pick(a.w);
@@ -257,7 +265,7 @@ __global__ __launch_bounds__(kThreads, 1) void gemm_kq_sp_kernel(const SpArgs a)
   const int16_t* __restrict__ ybs = a.ybs;
   const int64_t M = a.M;
   const int64_t m0 = (int64_t)mt * kBM;
-  const int64_t n0 = (int64_t)ct * kBN;
+  const int64_t n0 = (int64_t)ct * kCols;
   // this workgroup's super-blocks: splits split .. split + P - 1, each
   // plen super-blocks (nsb is a multiple of 2 S when S > 1)
   const int plen = nsb / S;
@@ -289,9 +297,21 @@ __global__ __launch_bounds__(kThreads, 1) void gemm_kq_sp_kernel(const SpArgs a)
   };
   // Q4_K keeps its three offsets; Q6_K forms its four at each use (from a
   // lane value the compiler cannot hoist), which keeps them out of registers
+  // GLU: the tile's four 32-row groups are gate, up, gate, up; copy i moves
+  // pieces 64 (i % 5) .. of group i / 5 (its fifth copy half a wave), so each
+  // reads one weight
   uint32_t woff[F::kWaveCopies];
 #pragma unroll
-  for (int u = 0; u < F::kWaveCopies; u++) woff[u] = Q6 ? 0u : woff_of(u, (uint32_t)lane);
+  for (int u = 0; u < F::kWaveCopies; u++) {
+    if constexpr (GLU >= 0) {
+      const uint32_t i = (uint32_t)(wv + 8 * u), f = 64u * (i % 5u) + (uint32_t)lane, grp = i / 5u;
+      const uint32_t row = f / 9u < 32u ? f / 9u : 31u;
+      const int64_t gc = n0 + 32 * (grp >> 1) + row < N ? n0 + 32 * (grp >> 1) + row : N - 1;
+      woff[u] = (uint32_t)gc * rowbytes + 16u * (f % 9u);
+    } else {
+      woff[u] = Q6 ? 0u : woff_of(u, (uint32_t)lane);
+    }
+  }
   // the per-super-block row inputs: bsums (32 bytes a row, 8 copies, one a
   // wave) and dy (4 bytes a row, 4 dword copies, waves 0-3)
   const uint32_t bsr = 32u * (uint32_t)wv + ((uint32_t)lane >> 1);
@@ -309,6 +329,11 @@ __global__ __launch_bounds__(kThreads, 1) void gemm_kq_sp_kernel(const SpArgs a)
       uint32_t ln = (uint32_t)lane;
       asm volatile("" : "+v"(ln));
       dma16(W + 16 * ((210 * (int64_t)sb) >> 4), woff_of(u, ln), lds_addr(sw + 1024 * i));
+    } else if constexpr (GLU >= 0) {
+      const int i = wv + 8 * u, c = i % 5;
+      if (i < 20 && (c < 4 || lane < 32))
+        dma16((const uint8_t*)((i / 5) & 1 ? a.w[1] : a.w[0]) + 144 * (int64_t)sb, woff[u],
+              lds_addr(sw + 4608 * (i / 5) + 1024 * c));
     } else if (wv + 8 * u < F::kCopies) {
       dma16(W + 144 * (int64_t)sb, woff[u], lds_addr(sw + 1024 * (wv + 8 * u)));
     }
@@ -629,6 +654,21 @@ __global__ __launch_bounds__(kThreads, 1) void gemm_kq_sp_kernel(const SpArgs a)
   // ---- store, the row factor undone (exact powers of two) ----
   float* __restrict__ dst = pick(a.dst);
   const int64_t ldd = pick(a.ldd);
+  if constexpr (GLU >= 0) {
+    const int64_t col = n0 + 32 * wn + r32;
+    if (col < N) {
+#pragma unroll
+      for (int tm = 0; tm < 2; tm++)
+#pragma unroll
+        for (int i = 0; i < 16; i++) {
+          const int lr = 64 * wm + 32 * tm + 8 * (i >> 2) + 4 * h + (i & 3);
+          const int64_t row = m0 + lr;
+          const float f = inv_pow2(s_rf[lr]);
+          if (row < M) dst[row * ldd + col] = glu_act<GLU>(acc[tm][0][i] * f * kOutScale, acc[tm][1][i] * f * kOutScale);
+        }
+    }
+    return;
+  }
   if (S == 1) {
 #pragma unroll
     for (int tn = 0; tn < 2; tn++) {
@@ -823,12 +863,45 @@ hipError_t launch_sp(const MvTargets& t, int64_t k, const ActPlanes& p, int64_t 
   if (units >= ((int64_t)1 << 31)) return hipErrorInvalidValue;
   a.remap = units % 8 == 0 ? 1 : 0;
   a.part = tiles > 0 ? (float*)split_ws : nullptr;
-  gemm_kq_sp_kernel<FMT><<<dim3((unsigned)units), kThreads, 0, st>>>(a);
+  gemm_kq_sp_kernel<FMT, -1><<<dim3((unsigned)units), kThreads, 0, st>>>(a);
   if (tiles > 0) {
     // unused entries past the last weight start at the end (no workgroups)
     for (int i = t.count; i < kMaxTargets; i++) a.tile_base[i] = tiles;
     gemm_q4k_sp_sum_kernel<<<dim3((unsigned)(tiles * kSumBlocksPerTile)), kSumThreads, 0, st>>>(a);
   }
+  return hipGetLastError();
+}
+
+hipError_t launch_gemm_q4k_sp_glu(int act, const void* w_gate, const void* w_up, int64_t n, int64_t k,
+                                  const ActPlanes& p, int64_t rows, float* dst, int64_t ldd, hipStream_t st) {
+  QMM_NOTE_LAUNCH();
+  SpArgs a{};
+  a.yq = p.codes;
+  a.yd = p.d;
+  a.ybs = (const int16_t*)p.sums;
+  a.M = rows;
+  a.nsb = (int)(k / 256);
+  a.mtiles = (int)((rows + kBM - 1) / kBM);
+  const int64_t units = (int64_t)a.mtiles * ((n + kBN / 2 - 1) / (kBN / 2));
+  if (units >= ((int64_t)1 << 31)) return hipErrorInvalidValue;
+  for (int i = 0; i < kMaxTargets; i++) {
+    a.w[i] = i == 0 ? w_gate : w_up;
+    a.dst[i] = dst;
+    a.ldd[i] = ldd;
+    a.n[i] = n;
+    a.splits[i] = a.per[i] = 1;
+    a.unit_end[i] = (int)units;
+  }
+  a.remap = units % 8 == 0 ? 1 : 0;
+  const dim3 grid((unsigned)units);
+  if (act == GLU_SILU)
+    gemm_kq_sp_kernel<T_Q4_K, GLU_SILU><<<grid, kThreads, 0, st>>>(a);
+  else if (act == GLU_SWIGLU_OAI)
+    gemm_kq_sp_kernel<T_Q4_K, GLU_SWIGLU_OAI><<<grid, kThreads, 0, st>>>(a);
+  else if (act == GLU_GELU)
+    gemm_kq_sp_kernel<T_Q4_K, GLU_GELU><<<grid, kThreads, 0, st>>>(a);
+  else
+    return hipErrorInvalidValue;
   return hipGetLastError();
 }
 

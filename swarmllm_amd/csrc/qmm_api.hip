@@ -868,6 +868,18 @@ int qmm_forward_glu(int type, int act, const void* w_gate, const void* w_up, con
     return status_of(qmm::launch_glu(act, parts[0], parts[1], qmm::gemm_kq_mid_splits(n, k, rows), dst, ldd, n, rows,
                                      st));
   }
+  // the single-pass GEMM, neither weight cut (together they have twice a
+  // weight's tiles): gate, up and the GLU in one launch
+  if (type == qmm::T_Q4_K && !g_force_dmmv.load(std::memory_order_relaxed) &&
+      sp_takes(type, w_gate, workspace, n, k, rows, st) && sp_takes(type, w_up, workspace, n, k, rows, st)) {
+    if (qmm::launch_act_quantize(layout, x, x_stride, k, rows, workspace, q8k_scale(), st) != hipSuccess)
+      return QMM_DEVICE_ERROR;
+    const qmm::ActPlanes p = qmm::act_planes(layout, workspace, k, rows);
+    if (qmm::launch_gemm_q4k_sp_glu(act, w_gate, w_up, n, k, p, rows, dst, ldd, st) != hipSuccess)
+      return QMM_DEVICE_ERROR;
+    g_gemm_launches.fetch_add(1, std::memory_order_relaxed);
+    return QMM_OK;
+  }
   float* gbuf = (float*)((char*)workspace + abytes);
   float* ubuf = (float*)((char*)gbuf + obytes);
   float* outs[2] = {gbuf, ubuf};

@@ -211,6 +211,10 @@ int gemm_q4k_sp_splits(int64_t n, int64_t k, int64_t rows, int cus);
 size_t gemm_q4k_sp_split_bytes(const MvTargets& t, int64_t k, int64_t rows, int cus);
 hipError_t launch_gemm_q4k_sp_targets(const MvTargets& t, int64_t k, const ActPlanes& p, int64_t rows, void* split_ws,
                                       size_t split_bytes, int cus, hipStream_t st);
+// act(x . gate) * (x . up) in one launch, neither weight cut: the bits of the
+// two products and launch_glu (act: glu_act.h).
+hipError_t launch_gemm_q4k_sp_glu(int act, const void* w_gate, const void* w_up, int64_t n, int64_t k,
+                                  const ActPlanes& p, int64_t rows, float* dst, int64_t ldd, hipStream_t st);
 // The same single-pass GEMM for Q6_K weights (k a multiple of 2048, from
 // gemm_q4k_sp_min_rows() rows): w8 = round(m_j (q - 32) / 256) with
 // m_j = round(127 sc_j / 16); same tiles, K splits and launches.
