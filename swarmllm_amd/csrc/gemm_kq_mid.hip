@@ -1,5 +1,5 @@
-// gemm_kq_mid.hip — Q4_K and Q6_K products of 17 to 128 activation rows on
-// the int8 matrix cores of gfx950: short prompts, large decode batches.
+// gemm_kq_mid.hip — Q4_K and Q6_K products of 17 to 128 activation rows (Q6_K
+// to 256) on the int8 matrix cores of gfx950: short prompts, large batches.
 //
 // dst[m][n] = sum over super-blocks of candle's Q4_K / Q6_K x Q8_K vec_dot
 // (vendor/candle/candle-core/src/quantized/k_quants.rs:2031-2111, 2598-2655)
@@ -22,16 +22,16 @@
 // weight rows) are both a few microseconds, while a tile that walks all of K
 // alone takes 2 us a super-block (the tiled GEMMs, uncut, at 77 rows: q, k, v
 // and o 36 us each, gate and up 39 each, the Q6_K down 110). So K is cut: a workgroup takes
-// 32 kNW weight rows, ALL activation rows (MT tiles of 32, so a weight byte is
-// read and expanded once) and one of S ranges of super-blocks; its partial
+// 128 weight rows, up to 96 activation rows (MT tiles of 32: below 97 rows a
+// weight byte is read and expanded once) and one of S ranges of super-blocks; its partial
 // goes to a slot and a second launch adds the slots in split order.
 //
-// Workgroup: kNW waves, each 32 weight rows x MT tiles of
+// Workgroup: 4 waves, each 32 weight rows x MT tiles of
 // v_mfma_i32_32x32x32_i8 (one MFMA per 32-value group, tile and operand).
 //   - The activation codes of a super-block (32 MT rows x 256 B, pieces
 //     XOR-swizzled by row) reach LDS by direct copies, one super-block ahead,
 //     double-buffered; the code sums (as f16) and dy through registers.
-//   - A wave's raw weight bytes (32 rows' blocks as their aligned 16-byte
+// //   - A wave's raw weight bytes weight bytes (32 rows' blocks as their aligned 16-byte
 //     pieces) are loaded one super-block ahead into registers, consecutive
 //     lanes on consecutive pieces, and written to the wave's own LDS slot
 //     when the current super-block is done; lanes read their row back.
@@ -40,8 +40,8 @@
 // Rows past M and weight rows past N are read as the last row (valid memory);
 // their outputs are never stored.
 //
-// Measured at 77 rows (an 8B layer, slots added in): q + k + v 24 us, o 19.5,
-// gate + up with its GLU 46, down 35; at 21 rows 15 / 13 / 28 / 26 (the
+// Measured at 77 rows (an 8B layer, slots added in): q + k + v 24 us, o 19,
+// gate + up with its GLU 45, down 34; at 21 rows 15 / 13 / 28 / 26 (the
 // two-row-tile few-row kernels before: 13 / 9 / 54 / 25). At 21 rows gate + up
 // reads HBM at 4.9 TB/s, 1.5 x its weight bytes (the 64-byte sector at each
 // 144-byte block's edges is fetched twice); at 77 the vector unit is busy 41%
@@ -77,6 +77,8 @@ __device__ __forceinline__ uint32_t pkmad(uint32_t a, uint32_t b, uint32_t c) {
                                                __builtin_bit_cast(u16x2, c)));
 }
 
+constexpr int kNW = 4, BN = 32 * kNW;  // waves of a workgroup, 32 weight rows each
+
 struct MidArgs {
   const void* w[kMaxTargets];
   float* dst[kMaxTargets];
@@ -90,6 +92,7 @@ struct MidArgs {
   const int16_t* ybs;
   float* part;  // null: uncut, a workgroup walks a tile's splits in turn
   int M, nsb, remap;
+  int chunks, per;  // row chunks of `per` rows (the last perhaps fewer)
 };
 
 template <int FMT>
@@ -102,14 +105,11 @@ struct MidFmt {
   static constexpr int kSlot = 32 * kStride + (kQ6 ? 16 : 0);
 };
 
-// kWide (97-128 rows): one set of integer accumulators, the high operand's
-// products first, then shifted, then the low operand's; the two sets of four
-// row tiles and their f32 sums would leave no registers for the rest.
-template <int FMT, int MT, int kNW, bool kWide>
+template <int FMT, int MT>
 __global__ __launch_bounds__(64 * kNW, 2) void gemm_kq_mid_kernel(const MidArgs a) {
   using F = MidFmt<FMT>;
   constexpr bool Q6 = F::kQ6;
-  constexpr int kRows = 32 * MT, BN = 32 * kNW, kThreads = 64 * kNW;
+  constexpr int kRows = 32 * MT, kThreads = 64 * kNW;
   constexpr int kACopies = 8 * MT / kNW;  // a wave's 1 KB activation copies a super-block
   static_assert(8 * MT % kNW == 0 && 2 * kRows <= kThreads, "copy shapes");
   __shared__ __attribute__((aligned(1024))) int8_t s_a[2][kRows * 256];
@@ -127,18 +127,21 @@ __global__ __launch_bounds__(64 * kNW, 2) void gemm_kq_mid_kernel(const MidArgs 
   const int idx = a.remap ? (b & 7) * (total >> 3) + (b >> 3) : b;
   const int t = idx < a.unit_end[0] ? 0 : idx < a.unit_end[1] ? 1 : idx < a.unit_end[2] ? 2 : 3;
   auto pick = [&](const auto& arr) { return t == 0 ? arr[0] : t == 1 ? arr[1] : t == 2 ? arr[2] : arr[3]; };
-  const int loc = idx - (t == 0 ? 0 : t == 1 ? a.unit_end[0] : t == 2 ? a.unit_end[1] : a.unit_end[2]);
+  const int loc0 = idx - (t == 0 ? 0 : t == 1 ? a.unit_end[0] : t == 2 ? a.unit_end[1] : a.unit_end[2]);
   const int64_t N = pick(a.n);
   const int S = pick(a.splits);
-  const int nsb = a.nsb, M = a.M;
+  const int nsb = a.nsb;
+  // the row chunk: consecutive workgroups share a weight tile
+  const int m0 = (loc0 % a.chunks) * a.per;
+  const int M = a.M - m0 < a.per ? a.M - m0 : a.per, loc = loc0 / a.chunks;
   const int ctiles = (int)((N + BN - 1) / BN);
   const bool cut = a.part != nullptr;
   const int ct = cut ? loc % ctiles : loc;
   const int s0 = cut ? loc / ctiles : 0, s1 = cut ? s0 + 1 : S;
   const uint8_t* __restrict__ W = (const uint8_t*)pick(a.w);
-  const int8_t* __restrict__ yq = a.yq;
-  const float* __restrict__ yd = a.yd;
-  const int16_t* __restrict__ ybs = a.ybs;
+  const int8_t* __restrict__ yq = a.yq + (int64_t)m0 * nsb * 256;
+  const float* __restrict__ yd = a.yd + (int64_t)m0 * nsb;
+  const int16_t* __restrict__ ybs = a.ybs + (int64_t)m0 * nsb * 16;
   const int64_t n0 = (int64_t)ct * BN;
   const uint32_t K = (uint32_t)nsb * 256u;
   const uint32_t rowbytes = (uint32_t)nsb * F::kBlock;
@@ -248,22 +251,31 @@ __global__ __launch_bounds__(64 * kNW, 2) void gemm_kq_mid_kernel(const MidArgs 
       h8 mb = {};
       float d = 0.0f, dmin = 0.0f;
       auto afrag = [&](int j, int m) -> i4v { return *(const i4v*)(sa + (fa0 ^ (32u * (uint32_t)j)) + 8192 * m); };
-      // one group's operands against every row tile; which: 1 high, 2 low, 3 both
-      auto mul = [&](int j, int which, const i4v& bh, const i4v& bl) {
+      // The eight 32-value groups, both operands, against every row tile. Group
+      // j + 1's operands are made under group j's MFMAs: a tile's activation
+      // fragment is read into its registers as soon as its MFMAs have issued.
+      auto groups = [&](auto&& prepare, auto&& build) {
         const i16v zero = {};
+        i4v af[MT], bh = {}, bl = {};
+        prepare(0);
 #pragma unroll
-        for (int m = 0; m < MT; m++) {
-          const i4v af = afrag(j, m);
-          if (which & 1) th[m] = __builtin_amdgcn_mfma_i32_32x32x32_i8(af, bh, j == 0 ? zero : th[m], 0, 0, 0);
-          if (which & 2)
-            tl[m] = __builtin_amdgcn_mfma_i32_32x32x32_i8(af, bl, j == 0 && !kWide ? zero : tl[m], 0, 0, 0);
+        for (int m = 0; m < MT; m++) af[m] = afrag(0, m);
+        build(0, bh, bl);
+#pragma unroll
+        for (int j = 0; j < 8; j++) {
+          i4v nh = {}, nl = {};
+          if (j < 7) prepare(j + 1);
+#pragma unroll
+          for (int m = 0; m < MT; m++) {
+            th[m] = __builtin_amdgcn_mfma_i32_32x32x32_i8(af[m], bh, j == 0 ? zero : th[m], 0, 0, 0);
+            tl[m] = __builtin_amdgcn_mfma_i32_32x32x32_i8(af[m], bl, j == 0 ? zero : tl[m], 0, 0, 0);
+            if (j < 7) af[m] = afrag(j + 1, m);
+          }
+          if (j < 7) build(j + 1, nh, nl);
+          bh = nh;
+          bl = nl;
+          if constexpr (MT > 1) __builtin_amdgcn_sched_barrier(0);
         }
-      };
-      auto widen = [&]() {  // kWide: the high products scaled, the low ones added to them
-#pragma unroll
-        for (int m = 0; m < MT; m++)
-#pragma unroll
-          for (int i = 0; i < 16; i++) tl[m][i] = (int)((uint32_t)th[m][i] << (Q6 ? 8 : 3));
       };
       if constexpr (!Q6) {
         const uint4 hdr = *(const uint4*)wrow;
@@ -284,77 +296,54 @@ __global__ __launch_bounds__(64 * kNW, 2) void gemm_kq_mid_kernel(const MidArgs 
           mb[2 * i] = v[0];
           mb[2 * i + 1] = v[1];
         }
-        auto sweep = [&](int which) {
+        uint4 raw[2];
+        auto prepare = [&](int j) {  // the codes of groups j, j + 1 (low and high nibbles)
+          if (j % 2 == 0) raw[(j >> 1) & 1] = *(const uint4*)(wrow + 16 + 16 * j + 16 * h);
+        };
+        auto build = [&](int j, i4v& bh, i4v& bl) {
+          const uint4& r = raw[(j >> 1) & 1];
+          const uint32_t rw[4] = {r.x, r.y, r.z, r.w};
+          const uint32_t sel = 0x0C000C00u + 0x00010001u * (uint32_t)(j & 3);
+          const uint32_t hj = __builtin_amdgcn_perm(0u, sh[j >> 2], sel);
+          const uint32_t lj = __builtin_amdgcn_perm(0u, sl[j >> 2], sel);
 #pragma unroll
-          for (int c = 0; c < 4; c++) {
-            const uint4 raw = *(const uint4*)(wrow + 16 + 32 * c + 16 * h);
-            const uint32_t rw[4] = {raw.x, raw.y, raw.z, raw.w};
-#pragma unroll
-            for (int p = 0; p < 2; p++) {
-              const int j = 2 * c + p;
-              const uint32_t sel = 0x0C000C00u + 0x00010001u * (uint32_t)(j & 3);
-              const uint32_t hj = __builtin_amdgcn_perm(0u, sh[j >> 2], sel);
-              const uint32_t lj = __builtin_amdgcn_perm(0u, sl[j >> 2], sel);
-              i4v bh = {}, bl = {};
-#pragma unroll
-              for (int e = 0; e < 4; e++) {
-                const uint32_t q = (p ? rw[e] >> 4 : rw[e]) & 0x0F0F0F0Fu;
-                if (which & 1) bh[e] = (int)pkmul(q, hj);
-                if (which & 2) bl[e] = (int)pkmul(q, lj);
-              }
-              mul(j, which, bh, bl);
-              if constexpr (MT > 2) __builtin_amdgcn_sched_barrier(0);
-            }
+          for (int e = 0; e < 4; e++) {
+            const uint32_t q = (j & 1 ? rw[e] >> 4 : rw[e]) & 0x0F0F0F0Fu;
+            bh[e] = (int)pkmul(q, hj);
+            bl[e] = (int)pkmul(q, lj);
           }
         };
-        if constexpr (kWide) {
-          sweep(1);
-          widen();
-          sweep(2);
-        } else {
-          sweep(3);
-        }
+        groups(prepare, build);
       } else {
         const int o = (int)((wbase + 210u * (uint32_t)sb) & 15u);
-        uint32_t scw[4];
+        uint32_t scw[4], ql[2][4], qh[4];
         lds_words<4>(wrow, o + 192, scw);
         d = 0.25f * h2f((uint16_t)lds_u16(wrow, o + 208));
-        auto sweep = [&](int which) {
+        auto prepare = [&](int j) {  // the code bytes of groups 4 (j / 4) .. + 3
+          if (j % 4 != 0) return;
+          const int hf = j >> 2;
+          lds_words<4>(wrow, o + 64 * hf + 16 * h, ql[0]);
+          lds_words<4>(wrow, o + 64 * hf + 32 + 16 * h, ql[1]);
+          lds_words<4>(wrow, o + 128 + 32 * hf + 16 * h, qh);
+        };
+        auto build = [&](int j, i4v& bh, i4v& bl) {
+          const int hf = j >> 2, gi = j & 3;
+          // scale of 16-value group 8 hf + 2 gi + h
+          const uint32_t sw = scw[2 * hf + (gi >> 1)];
+          const int sc = (int)(int8_t)((sw >> (16 * (gi & 1) + 8 * h)) & 0xFFu);
+          const uint32_t sc4 = ((uint32_t)(4 * sc) & 0xFFFFu) * 0x10001u;
+          const uint32_t kb = ((uint32_t)(128 - 128 * sc) & 0xFFFFu) * 0x10001u;
 #pragma unroll
-          for (int hf = 0; hf < 2; hf++) {
-            uint32_t ql[2][4], qh[4];
-            lds_words<4>(wrow, o + 64 * hf + 16 * h, ql[0]);
-            lds_words<4>(wrow, o + 64 * hf + 32 + 16 * h, ql[1]);
-            lds_words<4>(wrow, o + 128 + 32 * hf + 16 * h, qh);
-#pragma unroll
-            for (int gi = 0; gi < 4; gi++) {
-              // scale of 16-value group 8 hf + 2 gi + h
-              const uint32_t sw = scw[2 * hf + (gi >> 1)];
-              const int sc = (int)(int8_t)((sw >> (16 * (gi & 1) + 8 * h)) & 0xFFu);
-              const uint32_t sc4 = ((uint32_t)(4 * sc) & 0xFFFFu) * 0x10001u;
-              const uint32_t kb = ((uint32_t)(128 - 128 * sc) & 0xFFFFu) * 0x10001u;
-              i4v bh = {}, bl = {};
-#pragma unroll
-              for (int e = 0; e < 4; e++) {
-                const uint32_t q = ((ql[gi & 1][e] >> (4 * (gi >> 1))) & 0x0F0F0F0Fu) |
-                                   (((qh[e] >> (2 * gi)) & 0x03030303u) << 4);
-                const uint32_t pe = pkmad(q & 0x00FF00FFu, sc4, kb);
-                const uint32_t po = pkmad((q >> 8) & 0x00FF00FFu, sc4, kb);
-                if (which & 1) bh[e] = (int)__builtin_amdgcn_perm(po, pe, 0x07030501u);
-                if (which & 2) bl[e] = (int)(__builtin_amdgcn_perm(po, pe, 0x06020400u) ^ 0x80808080u);
-              }
-              mul(4 * hf + gi, which, bh, bl);
-              if constexpr (MT > 2) __builtin_amdgcn_sched_barrier(0);
-            }
+          for (int e = 0; e < 4; e++) {
+            const uint32_t q =
+                ((ql[gi & 1][e] >> (4 * (gi >> 1))) & 0x0F0F0F0Fu) | (((qh[e] >> (2 * gi)) & 0x03030303u) << 4);
+            const uint32_t pe = pkmad(q & 0x00FF00FFu, sc4, kb);
+            const uint32_t po = pkmad((q >> 8) & 0x00FF00FFu, sc4, kb);
+            bh[e] = (int)__builtin_amdgcn_perm(po, pe, 0x07030501u);
+            bl[e] = (int)(__builtin_amdgcn_perm(po, pe, 0x06020400u) ^ 0x80808080u);
           }
         };
-        if constexpr (kWide) {
-          sweep(1);
-          widen();
-          sweep(2);
-        } else {
-          sweep(3);
-        }
+        groups(prepare, build);
       }
       // acc += dy (d T - dmin Tm)
 #pragma unroll
@@ -368,7 +357,7 @@ __global__ __launch_bounds__(64 * kNW, 2) void gemm_kq_mid_kernel(const MidArgs 
 #pragma unroll
           for (int e = 0; e < 4; e++) {
             const int i = 4 * g + e;
-            const int tt = kWide ? tl[m][i] : (int)(((uint32_t)th[m][i] << (Q6 ? 8 : 3)) + (uint32_t)tl[m][i]);
+            const int tt = (int)(((uint32_t)th[m][i] << (Q6 ? 8 : 3)) + (uint32_t)tl[m][i]);
             float u;
             if constexpr (Q6)
               u = d * (float)tt;
@@ -389,7 +378,7 @@ __global__ __launch_bounds__(64 * kNW, 2) void gemm_kq_mid_kernel(const MidArgs 
     }
 
     if (col < N) {
-      float* __restrict__ out = cut ? a.part + pick(a.part_off) + (int64_t)s * M * N + col : dst + col;
+      float* __restrict__ out = cut ? a.part + pick(a.part_off) + ((int64_t)s * a.M + m0) * N + col : dst + m0 * ldd + col;
       int64_t ldo = cut ? N : ldd;
       int hrow = 4 * h;
       // the rows and their addresses are formed here, not kept live over the K loop
@@ -444,23 +433,22 @@ __global__ __launch_bounds__(256) void gemm_kq_mid_sum_kernel(const MidArgs a) {
   }
 }
 
-int tile_cols(int64_t rows) { return rows > 96 ? 256 : 128; }
-
-template <int FMT, int MT, int kNW, bool kWide>
-void launch_kernel(const MidArgs& a, int units, hipStream_t st) {
-  gemm_kq_mid_kernel<FMT, MT, kNW, kWide><<<dim3((unsigned)units), 64 * kNW, 0, st>>>(a);
+// Row chunks of at most 96 rows (three tiles: a fourth leaves too few registers
+// for the weights in flight), alike in size.
+int64_t chunk_rows(int64_t rows) {
+  const int64_t c = (rows + 95) / 96;
+  return (rows + c - 1) / c;
 }
 
 template <int FMT>
 void launch_fmt(const MidArgs& a, int units, hipStream_t st) {
-  if (a.M <= 32)
-    launch_kernel<FMT, 1, 4, false>(a, units, st);
-  else if (a.M <= 64)
-    launch_kernel<FMT, 2, 4, false>(a, units, st);
-  else if (a.M <= 96)
-    launch_kernel<FMT, 3, 4, false>(a, units, st);
+  const dim3 grid((unsigned)units);
+  if (a.per <= 32)
+    gemm_kq_mid_kernel<FMT, 1><<<grid, 64 * kNW, 0, st>>>(a);
+  else if (a.per <= 64)
+    gemm_kq_mid_kernel<FMT, 2><<<grid, 64 * kNW, 0, st>>>(a);
   else
-    launch_kernel<FMT, 4, 8, true>(a, units, st);
+    gemm_kq_mid_kernel<FMT, 3><<<grid, 64 * kNW, 0, st>>>(a);
 }
 
 }  // namespace
@@ -472,29 +460,36 @@ void launch_fmt(const MidArgs& a, int units, hipStream_t st) {
 // against 21.8 / 24.8, 14336 x 4096 22.5 / 23.5 against 23.9 / 29.2, 8192 x
 // 28672 57 / 61 against 64 / 79; Q6_K alike): it takes those of 14336 x 4096
 // values, below 24 rows only the wide ones and those over twice that.
+// Above 32 rows the tiled GEMMs keep rows of fewer than six super-blocks (1024
+// x 1024 at 64 rows: 15.0 us against 14.7 here for Q4_K, 14.4 against 16.0 for
+// Q6_K) and, past 96 rows, the Q6_K products that fill them (14336 x 4096 at
+// 128 rows 44 us against 48); past 128 rows it takes the Q6_K products the
+// single-pass GEMM leaves to the exact one (k no multiple of 2048): 4096 x
+// 11008 at 130 / 256 rows 45 / 75 us against 96 / 97.
 bool gemm_kq_mid_fits(int type, int64_t n, int64_t k, int64_t rows) {
   const int64_t block = type == T_Q4_K ? 144 : type == T_Q6_K ? 210 : 0;
   if (rows <= 32) {
     constexpr int64_t kLarge = (int64_t)14336 * 4096;
     if (n * k < kLarge || (rows < 24 && n < 14336 && n * k < 2 * kLarge)) return false;
+  } else if (k < 1536) {
+    return false;
   }
+  if (type == T_Q6_K && rows > 96 && n > 4096 && k < 8192) return false;
+  if (rows > 128 && (type != T_Q6_K || k % 2048 == 0 || rows > 256 || (rows > 192 && k < 4096))) return false;
   // 32-bit byte offsets inside the kernel
-  return block != 0 && rows >= kMidMinRows && rows <= kMidMaxRows && k % 256 == 0 &&
-         n * (k / 256) * block + 16 < ((int64_t)1 << 31) && 128 * k < ((int64_t)1 << 31) && n * rows < ((int64_t)1 << 31);
+  return block != 0 && rows >= kMidMinRows && k % 256 == 0 && n * (k / 256) * block + 16 < ((int64_t)1 << 31) &&
+         256 * k < ((int64_t)1 << 31) && n * rows < ((int64_t)1 << 31);
 }
 
 // K ranges of one weight's product, from its own shape (so a weight's bits do
 // not depend on the weights it shares a launch with): as many as bring its
-// workgroups to 256 (128 columns each, two on a CU: gate and up share a
-// launch, and 14336 x 4096 of either gives 224), at least 2 super-blocks a
-// range. Past 96 rows a CU holds one workgroup (256 columns): 128 for the wide
-// weights. Measured at 77 rows, gate + up / q + k + v / down of an 8B layer,
-// slots added: 128 workgroups 54 / 24 / 52 us, 256 45 / 24 / 35, 512 56 / 23 /
-// 36; at 128 rows with 128 / 256 wide workgroups 62 / 76 us for gate + up,
-// 67 / 50 for down.
+// workgroups to 256 (two fit a CU: gate and up share a launch, and 14336 x 4096
+// of either gives 224), at least 2 super-blocks a range. Measured at 77 rows,
+// gate + up / q + k + v / down of an 8B layer, slots added: 128 workgroups 54 /
+// 24 / 52 us, 256 45 / 24 / 35, 512 56 / 23 / 36.
 int gemm_kq_mid_splits(int64_t n, int64_t k, int64_t rows) {
-  const int64_t bn = tile_cols(rows), tiles = (n + bn - 1) / bn;
-  int64_t s = (bn == 256 && tiles > 32 ? 128 : 256) / tiles;
+  const int64_t tiles = (n + BN - 1) / BN * ((rows + 95) / 96);
+  int64_t s = 256 / tiles;
   const int64_t most = k / 512;
   if (s > most) s = most;
   if (s > 16) s = 16;
@@ -525,8 +520,9 @@ static hipError_t launch_mid(const MvTargets& t, int64_t k, const ActPlanes& p, 
   a.yd = p.d;
   a.ybs = (const int16_t*)p.sums;
   a.M = (int)rows;
+  a.per = (int)chunk_rows(rows);
+  a.chunks = (int)((rows + a.per - 1) / a.per);
   a.nsb = (int)(k / 256);
-  const int64_t bn = tile_cols(rows);
   int64_t units = 0, floats = 0, most = 0;
   for (int i = 0; i < kMaxTargets; i++) {
     const int j = i < t.count ? i : t.count - 1;  // unused entries repeat the last weight, with no units
@@ -538,7 +534,7 @@ static hipError_t launch_mid(const MvTargets& t, int64_t k, const ActPlanes& p, 
     a.splits[i] = gemm_kq_mid_splits(n, k, rows);
     a.part_off[i] = floats;
     if (i < t.count) {
-      units += (n + bn - 1) / bn * (cut ? a.splits[i] : 1);
+      units += (n + BN - 1) / BN * a.chunks * (cut ? a.splits[i] : 1);
       if (parts) parts[i] = (float*)slots + floats;
       floats += (int64_t)(align_up((size_t)(n * rows) * 4 * a.splits[i], 256) / 4);
       most = n * rows > most ? n * rows : most;

@@ -227,8 +227,8 @@ bool mmq_allows(int64_t rows) {
 
 bool aligned16(const void* p) { return ((uintptr_t)p & 15) == 0; }
 
-// Q4_K and Q6_K at 17-128 rows (gemm_kq_mid.hip): all activation rows in one
-// workgroup tile, the weight cut along K.
+// Q4_K and Q6_K at 17-128 rows and Q6_K's up to 256 that the single-pass GEMM
+// does not take (gemm_kq_mid.hip): the weight cut along K.
 bool mid_takes(int type, const void* w, const void* xq, int64_t n, int64_t k, int64_t rows) {
   return mmq_allows(rows) && aligned16(w) && aligned16(xq) && qmm::gemm_kq_mid_fits(type, n, k, rows);
 }
@@ -685,7 +685,7 @@ int qmm_forward_shared(int type, int count, const void* const* w, const int64_t*
   const int layout = qmm_act_layout(type, rows);
   const size_t bytes = qmm::act_bytes(layout, k, rows);
   const hipStream_t st = (hipStream_t)stream;
-  // the 17-128 row kernel's and the single-pass GEMM's products go
+  // the short-batch kernel's and the single-pass GEMM's products go
   // kMaxTargets to a launch; their split slots follow the activation (one
   // launch's worth, reused launch after launch)
   size_t split = 0;
@@ -832,7 +832,7 @@ int qmm_forward_glu(int type, int act, const void* w_gate, const void* w_up, con
   const size_t abytes = qmm::act_bytes(layout, k, rows);
   const size_t obytes = qmm::align_up((size_t)(rows * n) * 4, 256);
   const size_t bytes = abytes + 2 * obytes;
-  // at 17-128 rows the GLU adds the products' K-split slots itself, when the
+  // in the short-batch kernel's range the GLU adds the products' K-split slots itself, when the
   // workspace holds them
   const bool mid = mid_takes(type, w_gate, workspace, n, k, rows) && mid_takes(type, w_up, workspace, n, k, rows);
   const void* w[2] = {w_gate, w_up};

@@ -224,7 +224,8 @@ hipError_t launch_gemm_q6k_sp(const void* w, int64_t n, int64_t k, const ActPlan
 hipError_t launch_gemm_q6k_sp_targets(const MvTargets& t, int64_t k, const ActPlanes& p, int64_t rows, void* split_ws,
                                       size_t split_bytes, int cus, hipStream_t st);
 
-// Q4_K and Q6_K products of 17 to 128 rows (gemm_kq_mid.hip): exact int32
+// Q4_K and Q6_K products of 17 to 128 rows, Q6_K's to 256 where the
+// single-pass GEMM does not take them (gemm_kq_mid.hip): exact int32
 // super-block sums, each weight cut along K into gemm_kq_mid_splits ranges
 // (from its own shape). Bytes of the slots of a launch over `t` (0: no weight
 // is cut, unless `always`). The launch, with slots of that size: the partial
@@ -232,7 +233,7 @@ hipError_t launch_gemm_q6k_sp_targets(const MvTargets& t, int64_t k, const ActPl
 // order, or with `parts` (slots of the `always` size) the slots left to the
 // caller ([split][rows][n] at parts[i]); without them a workgroup adds a
 // tile's splits into dst one after another: the same bits.
-constexpr int kMidMinRows = 17, kMidMaxRows = 128;
+constexpr int kMidMinRows = 17;
 bool gemm_kq_mid_fits(int type, int64_t n, int64_t k, int64_t rows);
 int gemm_kq_mid_splits(int64_t n, int64_t k, int64_t rows);
 size_t gemm_kq_mid_slot_bytes(const MvTargets& t, int64_t k, int64_t rows, bool always);

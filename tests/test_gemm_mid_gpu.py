@@ -1,6 +1,6 @@
 """Q4_K and Q6_K products of 17-128 rows (gemm_kq_mid.hip) against the CPU
-oracle: at the edges of its row tiles (32, 64, 96, 128), of its column tiles
-(128, and 256 past 96 rows) and of its K cut, and with the largest codes and
+oracle: at the edges of its row tiles (32, 64, 96), of its row chunks
+(97, 129, 193 rows), of its 128-column tiles and of its K cut, and with the largest codes and
 scales a block can hold.
 
 Bound: the super-block sums are exact integers and the min sums exact f32, so
@@ -28,9 +28,11 @@ BOUND = 1e-5
 KERNEL = {qref.Q4_K: "launch_gemm_q4k_mid(", qref.Q6_K: "launch_gemm_q6k("}
 
 SHAPES = [  # (n, k, rows)
-    (129, 1024, 33), (1, 256, 40), (128, 768, 64), (300, 4096, 65), (2048, 2048, 96),
-    (255, 512, 97), (257, 2560, 128), (1024, 14336, 50), (9000, 512, 100),
+    (129, 1536, 33), (1, 1536, 40), (128, 1792, 64), (300, 4096, 65), (2048, 2048, 96), (255, 1536, 97),
+    (257, 2560, 128), (1024, 14336, 50), (9000, 1792, 100),
 ]
+# past 128 rows (two and three row chunks): Q6_K rows the single-pass GEMM does not take
+CHUNKED = [(300, 2816, 129), (257, 5632, 192), (130, 4352, 193), (1000, 11008, 256)]
 
 
 def stream():
@@ -48,8 +50,8 @@ def forward(t, qt, x, n, k, rows, ws_bytes=None):
     return out, need.value
 
 
-@pytest.mark.parametrize("t", [qref.Q4_K, qref.Q6_K], ids=["q4k", "q6k"])
-@pytest.mark.parametrize("n,k,rows", SHAPES)
+@pytest.mark.parametrize("t,n,k,rows", [(t, *s) for t in (qref.Q4_K, qref.Q6_K) for s in SHAPES]
+                         + [(qref.Q6_K, *s) for s in CHUNKED])
 def test_against_the_oracle_and_the_same_bits_whatever_the_workspace(t, n, k, rows):
     rng = np.random.default_rng(zlib.crc32(f"mid-{t}-{n}-{k}-{rows}".encode()))
     wq = qref.from_float(t, weights(rng, n, k))
