@@ -351,6 +351,38 @@ bool stream_supported(int type, int64_t k, int64_t rows) {
   return false;
 }
 
+// Whether the streaming kernel is the one for an activation whose planes are
+// made. A lane of it holds its part of a weight row and of the activation in
+// registers, which for Q4_K at 2 rows of more than 4096 values and 1 of more
+// than 8192 do not fit (up to 187 are spilled); the multi-row kernel reads the
+// planes from the caches (with their own launch: 1 row, 8192 x 11008 53 -> 15
+// us, 8192 x 16384 57 -> 20; 2 rows, 28672 x 8192 78 -> 36, 14336 x 5120 43
+// -> 19, 128 x 8192 12 -> 8).
+bool stream_from_planes(int type, int64_t k, int64_t rows) {
+  return stream_supported(type, k, rows) && (type != qmm::T_Q4_K || k <= (rows == 1 ? 8192 : 4096));
+}
+
+// Whether it also takes, quantizing the activation itself, these `count`
+// weights of n_total rows together. Where the multi-row kernel is faster, the
+// quantizer's launch and one a weight still cost the host 3.5 us each past
+// the first (a forward of one launch 14 us), so the streaming kernel keeps what it
+// does in under about 17 us: 1 row while a wave has one weight row (4096 x
+// 14336 17 us), 2 rows up to 3072 weight rows, and 2560 more for each further
+// weight. Without room for the planes it takes all that it supports.
+bool stream_takes(int type, int64_t k, int64_t n_total, int count, int64_t rows) {
+  return stream_from_planes(type, k, rows) ||
+         (stream_supported(type, k, rows) &&
+          n_total <= (int64_t)cu_count() * ((rows == 1 ? 16 : 12) + 10 * (count - 1)));
+}
+
+// The same of the launch that also applies the GLU, at 2 rows of more than
+// 4096 values, against the two products and the GLU in launches of their own
+// (4352 x 4352 78 -> 23 us, 13824 x 5120 157 -> 37, 28672 x 8192 287 -> 69;
+// four launches cost the host about 24 us).
+bool stream_glu_takes(int64_t k, int64_t n, int64_t rows) {
+  return rows == 1 || k <= 4096 || n <= (int64_t)cu_count() * 6;
+}
+
 // Launch shape of the Q4_K decode kernel for n_total weight rows, in 16-wave
 // workgroups (one activation fill per 16 waves): a row per wave up to 16
 // waves a CU; beyond that, about 1.5 rows per wave up to 32 waves a CU, the
@@ -563,7 +595,7 @@ int qmm_matvec(int type, const void* w, const void* xq, float* dst, int64_t ldd,
   const qmm::ActPlanes p = qmm::act_planes(layout, (void*)xq, k, rows);
   clear_stale_error();
   hipError_t e;
-  if (stream_supported(type, k, rows))
+  if (stream_from_planes(type, k, rows))
     e = launch_stream_targets(type, 1, &w, &n, &dst, &ldd, k, rows, nullptr, 0, &p, (hipStream_t)stream);
   else
     e = qmm::launch_matvec(type, w, n, k, p, rows, dst, ldd, (hipStream_t)stream);
@@ -603,7 +635,7 @@ int launch_product(int type, const void* w, int64_t n, int64_t k, const void* xq
     const int64_t nr = rows - r0 < step ? rows - r0 : step;
     const qmm::ActPlanes pr = qmm::act_rows(layout, p, k, r0);
     float* d = dst + r0 * ldd;
-    const hipError_t e = stream_supported(type, k, nr)
+    const hipError_t e = stream_from_planes(type, k, nr)
                              ? launch_stream_targets(type, 1, &w, &n, &d, &ldd, k, nr, nullptr, 0, &pr, st)
                              : qmm::launch_matvec(type, w, n, k, pr, nr, d, ldd, st);
     if (e != hipSuccess) return QMM_DEVICE_ERROR;
@@ -643,7 +675,7 @@ int qmm_forward(int type, const void* w, const float* x, int64_t x_stride, float
   clear_stale_error();
   if (g_force_dmmv.load(std::memory_order_relaxed))
     return status_of(qmm::launch_dmmv(type, w, n, k, x, x_stride, rows, dst, ldd, st));
-  if (stream_supported(type, k, rows) && qmm::mv_q4k_rows_fusable(x, x_stride) &&
+  if (stream_takes(type, k, n, 1, rows) && qmm::mv_q4k_rows_fusable(x, x_stride) &&
       !matrix_takes(type, w, workspace, n, k, rows, st)) {
     // the activation is quantized inside the product's own launch
     const hipError_t e = launch_stream_targets(type, 1, &w, &n, &dst, &ldd, k, rows, x, x_stride, nullptr, st);
@@ -728,7 +760,11 @@ int qmm_forward_shared(int type, int count, const void* const* w, const int64_t*
         return QMM_DEVICE_ERROR;
     return QMM_OK;
   }
-  bool fused = stream_supported(type, k, rows) && qmm::mv_q4k_rows_fusable(x, x_stride);
+  int64_t n_total = 0;
+  for (int i = 0; i < count; i++) n_total += n[i];
+  const bool room = workspace != nullptr && workspace_bytes >= bytes;
+  bool fused = (room ? stream_takes(type, k, n_total, count, rows) : stream_supported(type, k, rows)) &&
+               qmm::mv_q4k_rows_fusable(x, x_stride);
   for (int i = 0; fused && i < count; i++) fused = !matrix_takes(type, w[i], workspace, n[i], k, rows, st);
   if (fused) {
     // one launch per kMaxTargets weights, each quantizing the activation in LDS
@@ -847,6 +883,7 @@ int qmm_forward_glu(int type, int act, const void* w_gate, const void* w_up, con
   const hipStream_t st = (hipStream_t)stream;
   clear_stale_error();
   if (type == qmm::T_Q4_K && !g_force_dmmv.load(std::memory_order_relaxed) && qmm::mv_q4k_glu_supported(k, rows) &&
+      (stream_glu_takes(k, n, rows) || workspace == nullptr || workspace_bytes < bytes) &&
       qmm::mv_q4k_rows_fusable(x, x_stride) &&
       !matrix_takes(type, w_gate, workspace, n, k, rows, st) && !matrix_takes(type, w_up, workspace, n, k, rows, st)) {
     if (qmm::launch_mv_q4k_glu(act, w_gate, w_up, n, k, rows, x, x_stride, nullptr, q8k_scale(), dst, ldd,
