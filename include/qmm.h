@@ -103,9 +103,10 @@ int qmm_matvec(int type, const void *w, const void *xq, float *dst, int64_t ldd,
  * reference's few-rows policy (quantized/cuda.rs:775-839): the decode
  * kernels up to qmm_matvec_max_rows() rows; for Q4_K and Q6_K the few-row
  * int8 matrix-core kernels from 4 rows on weights of 2 MiB or more and for
- * 9-16 rows, the exact short-batch kernel for 17-128 rows, then the int8
- * matrix-core GEMMs; for Q8_0, IQ4_NL
- * and MXFP4 the int8 matrix-core GEMM from 9 rows. Nothing is allocated.
+ * 9-32 rows, the exact short-batch kernel to 128 rows (from 17 for weights
+ * of 14336 x 4096 values and more, from 33 for k >= 1536; Q6_K to 256 rows
+ * where k is no multiple of 2048), and the int8 matrix-core GEMMs past it;
+ * for Q8_0, IQ4_NL and MXFP4 the int8 matrix-core GEMM from 9 rows. Nothing is allocated.
  * The SWARMLLM_QMATMUL_MMQ switches below move these lines. Replaces
  * swarm_mmq_matmul's launch step (mmq_entry.cu:162-203), which multiplies
  * the activation swarm_mmq_quantize produced. */
@@ -215,7 +216,9 @@ size_t qmm_forward_noalloc_max_bytes(void);
  * activation is quantized once for all of them. Weight i has n[i] rows and
  * writes dst[i] with leading dimension ldd[i]. For Q4_K and Q6_K at 1-2
  * rows the products run as one launch per 4 weights, each quantizing the
- * activation in LDS (workspace unused); otherwise the activation is
+ * activation in LDS (workspace unused; Q4_K at 2 rows of more than 4096
+ * values or 1 of more than 8192 only for few weight rows or without room in
+ * the workspace); otherwise the activation is
  * quantized once into the workspace and each weight's product reads it, the
  * weights the few-row and short-batch matrix-core kernels or the single-pass
  * GEMMs take sharing one launch per 4 (each weight's K split as its own forward would
@@ -240,7 +243,8 @@ enum qmm_glu_act_id {
  * activation, and the gated activation between them, written once. For Q4_K
  * at 1-2 rows and k <= 8192 with a 16-byte aligned activation this is ONE
  * launch (each wave computes gate row j and up row j and writes the product;
- * the activation quantized in LDS), and past 128 rows one launch of the
+ * the activation quantized in LDS; at 2 rows and k > 4096 only for few weight
+ * rows or a workspace smaller than need), and past 128 rows one launch of the
  * single-pass GEMM, neither weight cut along K; otherwise the two products run
  * as qmm_forward_shared into the workspace, followed by the elementwise GLU.
  * The results equal the two products (uncut past 128 rows) followed by

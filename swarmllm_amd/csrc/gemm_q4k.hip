@@ -1,4 +1,6 @@
-// gemm_q4k.hip — Q4_K prefill GEMM on the int8 matrix cores of gfx950.
+// gemm_q4k.hip — Q4_K prefill GEMM on the int8 matrix cores of gfx950, from 33
+// activation rows what neither the short-batch kernel (gemm_kq_mid.hip) nor the
+// single pass (gemm_q4k_sp.hip) takes: rows of few super-blocks.
 //
 // dst[m][n] = sum over super-blocks sb of
 //     d_n dy_m * sum_j sc_nj * sum_{i in j} q_ni y_mi  -  dmin_n dy_m * sum_j m_nj * S_mj

@@ -1,5 +1,6 @@
 // gemm_q6k.hip — Q6_K prefill GEMM on the int8 matrix cores of gfx950, from
-// 33 activation rows (fewer: gemm_q6k_skinny.hip).
+// 33 activation rows (fewer: gemm_q6k_skinny.hip) what neither the short-batch
+// kernel (gemm_kq_mid.hip) nor the K-cut single pass (gemm_q4k_sp.hip) takes.
 //
 // dst[m][n] = sum over super-blocks of  d_n dy_m sum_g sc_ng sum_{i in g} (q_ni - 32) y_mi
 // is candle's Q6_K x Q8_K vec_dot (vendor/candle/candle-core/src/quantized/
