@@ -251,6 +251,21 @@ __global__ __launch_bounds__(256) void mv_b32_kernel(const uint8_t* __restrict__
 // ===========================================================================
 int matvec_max_rows() { return 8; }
 
+template <int NR, int RPW>
+static hipError_t launch_b32(int type, const uint8_t* W, int64_t n, int64_t k, const ActPlanes& p, float* dst,
+                             int64_t ldd, hipStream_t st) {
+  const int nb = (int)(k / 32);
+  const int64_t waves = (n + RPW - 1) / RPW;
+  const dim3 grid((unsigned)((waves + kWavesPerBlock - 1) / kWavesPerBlock));
+  switch (type) {
+    case T_Q8_0: mv_b32_kernel<T_Q8_0, NR, RPW><<<grid, 256, 0, st>>>(W, n, nb, p.codes, p.d, dst, ldd); break;
+    case T_IQ4_NL: mv_b32_kernel<T_IQ4_NL, NR, RPW><<<grid, 256, 0, st>>>(W, n, nb, p.codes, p.d, dst, ldd); break;
+    case T_MXFP4: mv_b32_kernel<T_MXFP4, NR, RPW><<<grid, 256, 0, st>>>(W, n, nb, p.codes, p.d, dst, ldd); break;
+    default: return hipErrorInvalidValue;
+  }
+  return hipGetLastError();
+}
+
 template <int NR>
 static hipError_t launch_nr(int type, const void* w, int64_t n, int64_t k, const ActPlanes& p, float* dst,
                             int64_t ldd, hipStream_t st) {
@@ -271,17 +286,17 @@ static hipError_t launch_nr(int type, const void* w, int64_t n, int64_t k, const
     }
     return hipGetLastError();
   }
-  const int nb = (int)(k / 32);
-  constexpr int RPW = NR <= 2 ? 2 : 1;
-  const int64_t waves = (n + RPW - 1) / RPW;
-  const dim3 grid((unsigned)((waves + kWavesPerBlock - 1) / kWavesPerBlock));
-  switch (type) {
-    case T_Q8_0: mv_b32_kernel<T_Q8_0, NR, RPW><<<grid, 256, 0, st>>>(W, n, nb, p.codes, p.d, dst, ldd); break;
-    case T_IQ4_NL: mv_b32_kernel<T_IQ4_NL, NR, RPW><<<grid, 256, 0, st>>>(W, n, nb, p.codes, p.d, dst, ldd); break;
-    case T_MXFP4: mv_b32_kernel<T_MXFP4, NR, RPW><<<grid, 256, 0, st>>>(W, n, nb, p.codes, p.d, dst, ldd); break;
-    default: return hipErrorInvalidValue;
-  }
-  return hipGetLastError();
+  // Past 2 activation rows the loads of the activation, as many a weight row
+  // as the weight's own times NR, weigh more than the weight's; two weight
+  // rows a wave share them where half the waves still fill the chip (8 rows,
+  // one or two weight rows a wave: Q8_0 14336 x 4096 59.4 / 47.0 us, 4096 x
+  // 14336 55.9 / 42.2, IQ4_NL 4096 x 4096 17.3 / 12.7, but Q8_0 1024 x 4096
+  // 9.0 / 11.4; 4 rows: IQ4_NL 14336 x 4096 29.9 / 25.0, but Q8_0 4096 x 14336
+  // 31.9 / 33.3).
+  if constexpr (NR <= 2) return launch_b32<NR, 2>(type, W, n, k, p, dst, ldd, st);
+  if constexpr (NR >= 4)
+    if (n >= (NR >= 7 ? 4096 : 8192)) return launch_b32<NR, 2>(type, W, n, k, p, dst, ldd, st);
+  return launch_b32<NR, 1>(type, W, n, k, p, dst, ldd, st);
 }
 
 hipError_t launch_matvec(int type, const void* w, int64_t n, int64_t k, const ActPlanes& p, int64_t rows, float* dst,
