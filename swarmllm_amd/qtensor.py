@@ -473,8 +473,9 @@ ACTIVATIONS = {"silu": _lib.GLU_SILU, "swiglu_oai": _lib.GLU_SWIGLU_OAI, "gelu":
 def forward_glu(xs: torch.Tensor, gate: "QMatMul", up: "QMatMul", activation: str = "silu") -> torch.Tensor:
     """act(xs · gateᵀ) * (xs · upᵀ): the gate and up products of an MLP sharing
     one quantized activation and the gated activation between them, written
-    once (qmm_forward_glu: one launch for Q4_K at 1-2 rows; otherwise the
-    shared products and the elementwise GLU). The reference's forward_block
+    once (qmm_forward_glu: one launch for Q4_K at 1-2 rows, long weight rows
+    at 2 rows aside, and for its prompts past 128 rows; otherwise the shared
+    products and the elementwise GLU). The reference's forward_block
     (src/inference/layers/mod.rs:583-632): forward_shared of ffn_up and
     ffn_gate, then silu_mul / swiglu_oai_mul / gelu(gate) * up."""
     if activation not in ACTIVATIONS:
