@@ -558,8 +558,8 @@ hipError_t launch_gemm_q4k_mid(const MvTargets& t, int64_t k, const ActPlanes& p
   return launch_mid<T_Q4_K>(t, k, p, rows, slots, slot_bytes, parts, st);
 }
 
-hipError_t launch_gemm_q6k(const MvTargets& t, int64_t k, const ActPlanes& p, int64_t rows, void* slots,
-                           size_t slot_bytes, float** parts, hipStream_t st) {
+hipError_t launch_gemm_q6k_mid(const MvTargets& t, int64_t k, const ActPlanes& p, int64_t rows, void* slots,
+                               size_t slot_bytes, float** parts, hipStream_t st) {
   QMM_NOTE_LAUNCH();
   return launch_mid<T_Q6_K>(t, k, p, rows, slots, slot_bytes, parts, st);
 }

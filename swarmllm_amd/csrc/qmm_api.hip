@@ -271,7 +271,7 @@ bool gemm_takes(int type, const void* w, const void* xq, int64_t n, int64_t k, i
 
 hipError_t launch_mid(int type, const qmm::MvTargets& t, int64_t k, const qmm::ActPlanes& p, int64_t rows, void* slots,
                       size_t slot_bytes, float** parts, hipStream_t st) {
-  return type == qmm::T_Q6_K ? qmm::launch_gemm_q6k(t, k, p, rows, slots, slot_bytes, parts, st)
+  return type == qmm::T_Q6_K ? qmm::launch_gemm_q6k_mid(t, k, p, rows, slots, slot_bytes, parts, st)
                              : qmm::launch_gemm_q4k_mid(t, k, p, rows, slots, slot_bytes, parts, st);
 }
 

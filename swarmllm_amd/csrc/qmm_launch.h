@@ -239,8 +239,8 @@ int gemm_kq_mid_splits(int64_t n, int64_t k, int64_t rows);
 size_t gemm_kq_mid_slot_bytes(const MvTargets& t, int64_t k, int64_t rows, bool always);
 hipError_t launch_gemm_q4k_mid(const MvTargets& t, int64_t k, const ActPlanes& p, int64_t rows, void* slots,
                                size_t slot_bytes, float** parts, hipStream_t st);
-hipError_t launch_gemm_q6k(const MvTargets& t, int64_t k, const ActPlanes& p, int64_t rows, void* slots,
-                           size_t slot_bytes, float** parts, hipStream_t st);
+hipError_t launch_gemm_q6k_mid(const MvTargets& t, int64_t k, const ActPlanes& p, int64_t rows, void* slots,
+                               size_t slot_bytes, float** parts, hipStream_t st);
 
 int gemm_q4k_min_rows();
 // The GEMM indexes with 32-bit byte offsets: the weight below 2 GiB and

@@ -1,7 +1,8 @@
 """The prefill GEMMs (int8 matrix cores) against the CPU oracle, through the
-C ABI: qmm_forward runs them for Q4_K weights from 33 rows (the two-pass
-kernel to 128 rows, the single-pass kernel from 129 rows at k >= 2048) and
-for Q6_K weights from 33 rows; the few-row kernels below 33.
+C ABI: qmm_forward runs them for Q4_K weights from 33 rows (the short-batch
+kernel to 128 rows, the single-pass kernel from 129 rows at k >= 2048, the
+two-pass kernel for shorter k) and for Q6_K weights from 33 rows; the few-row
+kernels below 33.
 
 Tolerance (for the MFMA GEMM): max
 |y_gpu - y_cpu| / (||w_j|| * ||x_r||) <= 2e-3. The GEMM multiplies the same
@@ -49,7 +50,7 @@ def activations(rng, rows: int, k: int, outliers: bool = False) -> np.ndarray:
 
 GEMM_SHAPES = [  # (k, n, rows): tails in M and N, one and many super-blocks
     (256, 128, 9), (256, 7, 9), (1024, 200, 16), (4096, 300, 33), (2560, 96, 64),
-    (4096, 1000, 130), (14336, 136, 40), (512, 384, 257),
+    (4096, 1000, 130), (14336, 136, 40), (512, 384, 257), (1280, 129, 77), (1792, 257, 200),
 ]
 
 
@@ -495,8 +496,17 @@ Q6K_GEMM_SHAPES = [  # (k, n, rows): one and many super-blocks; rows of 3, 5, 12
     # every even offset of their windows) and of 8 and 56 (the same offset in every row); row and
     # weight-row tails; 4- and 8-wave tiles; the XCD remap (tiles % 8 == 0) and without it
     (256, 70, 33), (768, 300, 40), (1280, 129, 97), (2048, 64, 200), (3072, 4100, 129),
-    (4096, 1000, 300), (14336, 256, 64), (2048, 2048, 512),
+    (4096, 1000, 300), (14336, 256, 64), (2048, 2048, 512), (2048, 4100, 97), (14592, 64, 257),
 ]
+
+
+def q6k_kernel(k, n, rows):
+    """The kernel of a Q6_K product past 32 rows, at these tests' sizes: the
+    single pass, the short-batch kernel or the tiled GEMM."""
+    if rows >= 129 and k % 2048 == 0:
+        return "launch_gemm_q6k_sp"
+    short = rows <= (128 if k % 2048 == 0 else 192) and k >= 1536 and (n <= 4096 or rows <= 96)
+    return "launch_gemm_q6k_mid(" if short else "launch_gemm_q6k("
 
 
 @pytest.mark.parametrize("k,n,rows", Q6K_GEMM_SHAPES)
@@ -511,7 +521,7 @@ def test_q6k_gemm_parity(k, n, rows):
     assert L.qmm_gemm_launches() == before + 1, "the MFMA GEMM did not run"
     kernel = L.qmm_last_kernel().decode()
     single_pass = rows >= 129 and k % 2048 == 0
-    assert ("launch_gemm_q6k_sp" if single_pass else "launch_gemm_q6k(") in kernel, kernel
+    assert q6k_kernel(k, n, rows) in kernel, kernel
     want = qref.matmul(qref.Q6_K, x, wq, n)
     wdeq = qref.to_float(qref.Q6_K, wq, n * k).reshape(n, k)
     err = normalised_error(y, want, wdeq, x)
@@ -519,14 +529,15 @@ def test_q6k_gemm_parity(k, n, rows):
     assert err <= (TIGHT_SP if single_pass else TIGHT_Q6K), f"k={k} n={n} rows={rows}: {err}"
 
 
-def test_q6k_gemm_special_activation_rows():
+@pytest.mark.parametrize("k,n,rows", [(2048, 96, 48), (2048, 4100, 97), (1280, 96, 48)])
+def test_q6k_gemm_special_activation_rows(k, n, rows):
     """The quantizer's edge-case rows (zeros, a constant, one outlier, ties,
     subnormal values, one-signed runs, near powers of two), rows scaled by
     1e-30 and 1e30, against extreme group scales (a weight row with one
-    large value per group)."""
+    large value per group): on the short-batch kernel (the first shape) and on
+    the tiled GEMM."""
     from helpers import special_rows
 
-    k, n, rows = 2048, 96, 48
     rng = np.random.default_rng(92)
     w = weights(rng, n, k)
     w[5, ::16] = 3.0  # each group's scale -128 or 127 next to small codes
@@ -538,7 +549,7 @@ def test_q6k_gemm_special_activation_rows():
     x[len(sp)] *= np.float32(1e-30)
     x[len(sp) + 1] *= np.float32(1e30)
     y = QMatMul(qt).forward(upload(x)).cpu().numpy()
-    assert "launch_gemm_q6k(" in lib().qmm_last_kernel().decode()
+    assert q6k_kernel(k, n, rows) in lib().qmm_last_kernel().decode()
     assert np.all(y[0] == 0.0) and np.all(y[:, 6] == 0.0)
     want = qref.matmul(qref.Q6_K, x, wq, n)
     wdeq = qref.to_float(qref.Q6_K, wq, n * k).reshape(n, k)
