@@ -281,13 +281,18 @@ bool matrix_takes(int type, const void* w, const void* xq, int64_t n, int64_t k,
          skinny_takes(type, w, xq, n, k, rows, st);
 }
 
+// One more weight of a launch (at most kMaxTargets).
+void add_target(qmm::MvTargets& t, const void* w, int64_t n, float* dst, int64_t ldd) {
+  const int i = t.count++;
+  t.w[i] = w;
+  t.dst[i] = dst;
+  t.ldd[i] = ldd;
+  t.row_end[i] = n + (i ? t.row_end[i - 1] : 0);
+}
+
 qmm::MvTargets one_target(const void* w, int64_t n, float* dst, int64_t ldd) {
   qmm::MvTargets t{};
-  t.w[0] = w;
-  t.dst[0] = dst;
-  t.ldd[0] = ldd;
-  t.row_end[0] = n;
-  t.count = 1;
+  add_target(t, w, n, dst, ldd);
   return t;
 }
 
@@ -332,14 +337,7 @@ hipError_t launch_sp(int type, const qmm::MvTargets& t, int64_t k, const qmm::Ac
 qmm::MvTargets targets_of(const void* const* w, const int64_t* n, float* const* dst, const int64_t* ldd, int i0,
                           int count) {
   qmm::MvTargets t{};
-  int64_t end = 0;
-  for (int i = i0; i < count && t.count < qmm::kMaxTargets; i++) {
-    t.w[t.count] = w[i];
-    t.dst[t.count] = dst[i];
-    t.ldd[t.count] = ldd[i];
-    end += n[i];
-    t.row_end[t.count++] = end;
-  }
+  for (int i = i0; i < count && t.count < qmm::kMaxTargets; i++) add_target(t, w[i], n[i], dst[i], ldd[i]);
   return t;
 }
 
@@ -620,13 +618,7 @@ int launch_product(int type, const void* w, int64_t n, int64_t k, const void* xq
     return QMM_OK;
   }
   if (skinny_takes(type, w, xq, n, k, rows, st)) {
-    qmm::MvTargets t{};
-    t.w[0] = w;
-    t.dst[0] = dst;
-    t.ldd[0] = ldd;
-    t.row_end[0] = n;
-    t.count = 1;
-    if (launch_skinny(type, t, k, p, rows, st) != hipSuccess) return QMM_DEVICE_ERROR;
+    if (launch_skinny(type, one_target(w, n, dst, ldd), k, p, rows, st) != hipSuccess) return QMM_DEVICE_ERROR;
     g_gemm_launches.fetch_add(1, std::memory_order_relaxed);
     return QMM_OK;
   }
@@ -717,34 +709,27 @@ int qmm_forward_shared(int type, int count, const void* const* w, const int64_t*
   const int layout = qmm_act_layout(type, rows);
   const size_t bytes = qmm::act_bytes(layout, k, rows);
   const hipStream_t st = (hipStream_t)stream;
-  // the short-batch kernel's and the single-pass GEMM's products go
-  // kMaxTargets to a launch; their split slots follow the activation (one
-  // launch's worth, reused launch after launch)
+  // the short-batch kernel's weights share its launches, kMaxTargets each, and
+  // so do those of the single-pass GEMM; their split slots follow the
+  // activation (one launch's worth, reused launch after launch)
+  auto mid_i = [&](int i) { return mid_takes(type, w[i], workspace, n[i], k, rows); };
+  auto sp_i = [&](int i) { return !mid_i(i) && sp_takes(type, w[i], workspace, n[i], k, rows, st); };
   size_t split = 0;
-  bool mid = true;  // the rows and type decide, and the weights' sizes and alignment
-  for (int i = 0; i < count; i++) mid = mid && mid_takes(type, w[i], workspace, n[i], k, rows);
-  for (int i0 = 0; mid && i0 < count; i0 += qmm::kMaxTargets) {
-    const size_t b = qmm::gemm_kq_mid_slot_bytes(targets_of(w, n, dst, ldd, i0, count), k, rows, false);
-    split = b > split ? b : split;
-  }
-  if (!mid) {
-    qmm::MvTargets g{};
-    int64_t end = 0;
-    for (int i = 0; i <= count; i++) {
-      if (i < count && sp_takes(type, w[i], workspace, n[i], k, rows, st)) {
-        g.w[g.count] = w[i];
-        g.dst[g.count] = dst[i];
-        g.ldd[g.count] = ldd[i];
-        end += n[i];
-        g.row_end[g.count] = end;
-        g.count++;
-      }
-      if (g.count == qmm::kMaxTargets || (i == count && g.count > 0)) {
-        const size_t b = qmm::gemm_q4k_sp_split_bytes(g, k, rows, (int)cu_count());
-        split = b > split ? b : split;
-        g = qmm::MvTargets{};
-        end = 0;
-      }
+  qmm::MvTargets midg{}, spg{};
+  for (int i = 0; i <= count; i++) {
+    if (i < count && mid_i(i))
+      add_target(midg, w[i], n[i], dst[i], ldd[i]);
+    else if (i < count && sp_i(i))
+      add_target(spg, w[i], n[i], dst[i], ldd[i]);
+    if (midg.count == qmm::kMaxTargets || (i == count && midg.count > 0)) {
+      const size_t b = qmm::gemm_kq_mid_slot_bytes(midg, k, rows, false);
+      split = b > split ? b : split;
+      midg = qmm::MvTargets{};
+    }
+    if (spg.count == qmm::kMaxTargets || (i == count && spg.count > 0)) {
+      const size_t b = qmm::gemm_q4k_sp_split_bytes(spg, k, rows, (int)cu_count());
+      split = b > split ? b : split;
+      spg = qmm::MvTargets{};
     }
   }
   *need = split ? qmm::align_up(bytes, 256) + split : bytes;
@@ -782,16 +767,6 @@ int qmm_forward_shared(int type, int count, const void* const* w, const int64_t*
   if (qmm::launch_act_quantize(layout, x, x_stride, k, rows, workspace, q8k_scale(), st) != hipSuccess)
     return QMM_DEVICE_ERROR;
   const qmm::ActPlanes p = qmm::act_planes(layout, workspace, k, rows);
-  if (mid) {
-    void* slots = split && workspace_bytes >= *need ? (char*)workspace + qmm::align_up(bytes, 256) : nullptr;
-    for (int i0 = 0; i0 < count; i0 += qmm::kMaxTargets) {
-      if (launch_mid(type, targets_of(w, n, dst, ldd, i0, count), k, p, rows, slots, slots ? split : 0, nullptr, st) !=
-          hipSuccess)
-        return QMM_DEVICE_ERROR;
-      g_gemm_launches.fetch_add(1, std::memory_order_relaxed);
-    }
-    return QMM_OK;
-  }
   if (!is_kquant(type)) {
     bool gemm = true;
     for (int i = 0; i < count; i++) gemm = gemm && gemm_takes(type, w[i], workspace, n[i], k, rows, st);
@@ -804,56 +779,43 @@ int qmm_forward_shared(int type, int count, const void* const* w, const int64_t*
       return QMM_OK;
     }
   }
-  // the weights the skinny kernel takes share its launches (kMaxTargets
-  // each), and so do those the single-pass GEMM takes
-  qmm::MvTargets grp{}, spg{};
-  int64_t end = 0, spend = 0;
-  auto flush = [&]() -> int {
-    if (grp.count == 0) return QMM_OK;
-    if (launch_skinny(type, grp, k, p, rows, st) != hipSuccess) return QMM_DEVICE_ERROR;
-    g_gemm_launches.fetch_add(1, std::memory_order_relaxed);
-    grp = qmm::MvTargets{};
-    end = 0;
-    return QMM_OK;
-  };
+  // the weights each of the short-batch, single-pass and few-row kernels takes
+  // share its launches
+  qmm::MvTargets grp{};
   const size_t off = qmm::align_up(bytes, 256);
   void* sws = workspace_bytes > off ? (char*)workspace + off : nullptr;
   const size_t sbytes = workspace_bytes > off ? workspace_bytes - off : 0;
-  auto flush_sp = [&]() -> int {
-    if (spg.count == 0) return QMM_OK;
-    if (launch_sp(type, spg, k, p, rows, sws, sbytes, st) != hipSuccess)
-      return QMM_DEVICE_ERROR;
+  auto flush = [&](qmm::MvTargets& t, auto&& launch_group) -> bool {
+    if (t.count == 0) return true;
+    if (launch_group(t) != hipSuccess) return false;
     g_gemm_launches.fetch_add(1, std::memory_order_relaxed);
-    spg = qmm::MvTargets{};
-    spend = 0;
-    return QMM_OK;
+    t = qmm::MvTargets{};
+    return true;
   };
-  const bool sp_ok = type == qmm::T_Q4_K || split == 0 || workspace_bytes >= *need;
+  auto mid_group = [&](const qmm::MvTargets& t) {
+    return launch_mid(type, t, k, p, rows, split ? sws : nullptr, split ? sbytes : 0, nullptr, st);
+  };
+  auto sp_group = [&](const qmm::MvTargets& t) { return launch_sp(type, t, k, p, rows, sws, sbytes, st); };
+  auto few_group = [&](const qmm::MvTargets& t) { return launch_skinny(type, t, k, p, rows, st); };
+  const bool room_split = split == 0 || workspace_bytes >= *need;
   for (int i = 0; i < count; i++) {
-    if (sp_ok && sp_takes(type, w[i], workspace, n[i], k, rows, st)) {
-      spg.w[spg.count] = w[i];
-      spg.dst[spg.count] = dst[i];
-      spg.ldd[spg.count] = ldd[i];
-      spend += n[i];
-      spg.row_end[spg.count] = spend;
-      if (++spg.count == qmm::kMaxTargets && flush_sp() != QMM_OK) return QMM_DEVICE_ERROR;
-      continue;
+    const bool mid = mid_i(i);
+    if (mid && room_split) {
+      add_target(midg, w[i], n[i], dst[i], ldd[i]);
+      if (midg.count == qmm::kMaxTargets && !flush(midg, mid_group)) return QMM_DEVICE_ERROR;
+    } else if (!mid && (type == qmm::T_Q4_K || room_split) && sp_i(i)) {
+      add_target(spg, w[i], n[i], dst[i], ldd[i]);
+      if (spg.count == qmm::kMaxTargets && !flush(spg, sp_group)) return QMM_DEVICE_ERROR;
+    } else if (!mid && !gemm_takes(type, w[i], workspace, n[i], k, rows, st) &&
+               skinny_takes(type, w[i], workspace, n[i], k, rows, st)) {
+      add_target(grp, w[i], n[i], dst[i], ldd[i]);
+      if (grp.count == qmm::kMaxTargets && !flush(grp, few_group)) return QMM_DEVICE_ERROR;
+    } else {
+      const int r = launch_product(type, w[i], n[i], k, workspace, p, layout, rows, dst[i], ldd[i], st);
+      if (r != QMM_OK) return r;
     }
-    if (!gemm_takes(type, w[i], workspace, n[i], k, rows, st) &&
-        skinny_takes(type, w[i], workspace, n[i], k, rows, st)) {
-      grp.w[grp.count] = w[i];
-      grp.dst[grp.count] = dst[i];
-      grp.ldd[grp.count] = ldd[i];
-      end += n[i];
-      grp.row_end[grp.count] = end;
-      if (++grp.count == qmm::kMaxTargets && flush() != QMM_OK) return QMM_DEVICE_ERROR;
-      continue;
-    }
-    const int r = launch_product(type, w[i], n[i], k, workspace, p, layout, rows, dst[i], ldd[i], st);
-    if (r != QMM_OK) return r;
   }
-  if (flush_sp() != QMM_OK) return QMM_DEVICE_ERROR;
-  return flush();
+  return flush(midg, mid_group) && flush(spg, sp_group) && flush(grp, few_group) ? QMM_OK : QMM_DEVICE_ERROR;
 }
 
 int qmm_forward_glu(int type, int act, const void* w_gate, const void* w_up, const float* x, int64_t x_stride,

@@ -77,6 +77,26 @@ def test_forward_plans_without_a_device_and_rejects_bad_shapes():
     assert L.qmm_matvec(12, None, None, None, 8, 256, 8, L.qmm_matvec_max_rows() + 1, 0) == _lib.QMM_UNSUPPORTED
 
 
+@pytest.mark.parametrize("t,k,ns,rows", [(12, 8192, (8192, 2048, 2048), 24), (12, 8192, (2048, 8192, 2048), 32),
+                                         (14, 8192, (8192, 2048, 2048), 24), (14, 5120, (5120, 1024, 1024), 100)])
+def test_shared_plan_counts_the_slots_of_the_weights_that_are_cut(t, k, ns, rows):
+    """Where the short-batch kernel takes only some of the weights (the large
+    one at 24-32 rows, the narrow ones at 100), the plan holds their K-split
+    slots: at least those of each weight's own forward."""
+    L = lib()
+    need, own = ctypes.c_size_t(0), ctypes.c_size_t(0)
+    act = L.qmm_act_bytes(_lib.ACT_Q8K, k, rows)
+    ptrs = (ctypes.c_void_p * 3)()
+    n = (ctypes.c_int64 * 3)(*ns)
+    assert L.qmm_forward_shared(t, 3, ptrs, n, ptrs, n, None, k, None, 0, ctypes.byref(need), k, rows, 0, 0) == 0
+    cut = []
+    for i in ns:
+        assert L.qmm_forward(t, None, None, k, None, i, None, 0, ctypes.byref(own), k, i, rows, 0, 0) == 0
+        cut.append(own.value > act)
+        assert need.value >= own.value
+    assert any(cut) and not all(cut)  # a mixed set
+
+
 def test_moe_plans_without_a_device_and_rejects_bad_routing_shapes():
     L = lib()
     need = ctypes.c_size_t(0)

@@ -18,7 +18,7 @@ import torch
 
 from helpers import normalised_error, special_rows, weights
 from oracle import qref
-from swarmllm_amd import GgmlDType, QMatMul, QTensor, _lib
+from swarmllm_amd import GgmlDType, QMatMul, QTensor, _lib, fill_normal
 from swarmllm_amd._lib import lib
 from swarmllm_amd.qtensor import quantize_act
 
@@ -85,8 +85,6 @@ LARGE = [  # up to 32 rows: the sizes the few-row kernels leave (n, k, rows, tak
 @pytest.mark.parametrize("t", [qref.Q4_K, qref.Q6_K], ids=["q4k", "q6k"])
 @pytest.mark.parametrize("n,k,rows,taken", LARGE)
 def test_large_weights_up_to_32_rows(t, n, k, rows, taken):
-    from swarmllm_amd import fill_normal
-
     qt = QTensor.quantize(fill_normal(n * k, seed=n + k, std=0.02).reshape(n, k), GgmlDType(t))
     xt = fill_normal(rows * k, seed=rows).reshape(rows, k)
     print(f"t={t} n={n} k={k} rows={rows}", flush=True)
@@ -111,6 +109,27 @@ def test_shared_products_keep_each_weights_bits(rows):
     x = torch.from_numpy(np.random.default_rng(9).standard_normal((rows, k)).astype(np.float32)).cuda()
     for m, y in zip(mats, QMatMul.forward_shared(x, mats)):
         assert torch.equal(y, m.forward(x))
+
+
+@pytest.mark.parametrize("t,k,ns,rows,launches", [
+    (qref.Q4_K, 8192, (8192, 2048, 2048), 24, 2), (qref.Q4_K, 8192, (2048, 8192, 2048), 32, 2),
+    (qref.Q6_K, 8192, (8192, 2048, 2048), 32, 2), (qref.Q6_K, 5120, (1024, 5120, 1024), 100, 2),
+])
+def test_sets_of_which_only_some_weights_are_taken(t, k, ns, rows, launches):
+    """Each kernel's weights share its launch (the short-batch kernel's with
+    their slots) and keep their own forward's bits."""
+    mats = [QMatMul(QTensor.quantize(fill_normal(n * k, seed=40 + i, std=0.02).reshape(n, k), GgmlDType(t)))
+            for i, n in enumerate(ns)]
+    x = fill_normal(rows * k, seed=rows).reshape(rows, k)
+    print(f"t={t} {ns} x {k} rows={rows}", flush=True)
+    before = lib().qmm_gemm_launches()
+    ys = QMatMul.forward_shared(x, mats)
+    assert lib().qmm_gemm_launches() == before + launches
+    kernels = set()
+    for m, y in zip(mats, ys):
+        assert torch.equal(y, m.forward(x))
+        kernels.add(KERNEL[t] in lib().qmm_last_kernel().decode())
+    assert kernels == {True, False}
 
 
 @pytest.mark.parametrize("rows", [40, 128])
