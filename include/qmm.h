@@ -106,7 +106,10 @@ int qmm_matvec(int type, const void *w, const void *xq, float *dst, int64_t ldd,
  * 9-32 rows, the exact short-batch kernel to 128 rows (from 17 for weights
  * of 14336 x 4096 values and more, from 33 for k >= 1536; Q6_K to 256 rows
  * where k is no multiple of 2048), and the int8 matrix-core GEMMs past it;
- * for Q8_0, IQ4_NL and MXFP4 the int8 matrix-core GEMM from 9 rows. Nothing is allocated.
+ * for Q8_0, IQ4_NL and MXFP4 the int8 matrix-core GEMM from 9 rows. Nothing is
+ * allocated, so a product that qmm_forward cuts along K into workspace slots
+ * runs uncut here, at 17-128 rows on the few-row kernels (32 rows a launch) or
+ * the Q6_K GEMM where they are faster: 1.1 to 3 times qmm_forward's time.
  * The SWARMLLM_QMATMUL_MMQ switches below move these lines. Replaces
  * swarm_mmq_matmul's launch step (mmq_entry.cu:162-203), which multiplies
  * the activation swarm_mmq_quantize produced. */
@@ -186,7 +189,8 @@ int qmm_accumulate_in_f32(int type);
  * most half the CUs, and for Q4_K and Q6_K at 17-128 rows, *need also counts
  * the slots of a K split (the product cut into parts along K, added in part
  * order); with a workspace that holds the activation but not those slots the
- * product runs uncut (at 17-128 rows with the same bits).
+ * product runs uncut, at 17-128 rows as exactly but in another order of sums
+ * and slower (as qmm_matmul, which has no slots).
  * Replaces the plan/launch pair of swarm_mmq_matmul (mmq_entry.cu:162-203). */
 int qmm_forward(int type, const void *w, const float *x, int64_t x_stride, float *dst, int64_t ldd,
                 void *workspace, size_t workspace_bytes, size_t *need, int64_t k, int64_t n, int64_t rows,

@@ -49,9 +49,9 @@
 // plain ones took 50 us at 21 rows, 62 at 77. A second super-block of
 // weights in flight changed nothing.
 //
-// A product's bits do not depend on the workspace: without room for the
-// slots one workgroup computes a tile's splits one after another and adds
-// each to dst, the same sums in the same order.
+// Without room for the slots one workgroup computes a tile's splits one after
+// another and adds each to dst, the same sums in the same order (a route for
+// the products no other kernel runs faster then: launch_mid_without_slots).
 #include "lds_copy.h"
 #include "mv_common.h"
 #include "qmm_device.h"

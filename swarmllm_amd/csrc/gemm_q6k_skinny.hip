@@ -358,14 +358,13 @@ hipError_t launch_q6(const MvTargets& t, int nsb, const ActPlanes& p, int64_t ro
 
 bool gemm_q6k_skinny_fits(int64_t k, int64_t rows) { return k % 256 == 0 && rows >= 1 && rows <= 32; }
 
-hipError_t launch_gemm_q6k_skinny(const MvTargets& t, int64_t k, const ActPlanes& p, int64_t rows, int cus,
+hipError_t launch_gemm_q6k_skinny(const MvTargets& t, int64_t k, const ActPlanes& p, int64_t rows, bool exact,
                                   hipStream_t st) {
-  (void)cus;
   const int nsb = (int)(k / 256);
   // the single-product form from k = 2048 (its rounding stays well inside
   // the 2e-3 bound there); shorter rows, and every row under
   // SWARMLLM_QMATMUL_EXACT, keep the exact form
-  if (k >= 2048 && !exact_forms()) {
+  if (k >= 2048 && !exact) {
     if (rows <= 16) return launch_q6<1, 1, 4, true>(t, nsb, p, rows, st);
     return launch_q6<2, 1, 4, true>(t, nsb, p, rows, st);
   }

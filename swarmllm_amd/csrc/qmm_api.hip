@@ -250,8 +250,8 @@ bool skinny_takes(int type, const void* w, const void* xq, int64_t n, int64_t k,
 }
 
 hipError_t launch_skinny(int type, const qmm::MvTargets& t, int64_t k, const qmm::ActPlanes& p, int64_t rows,
-                         hipStream_t st) {
-  if (type == qmm::T_Q6_K) return qmm::launch_gemm_q6k_skinny(t, k, p, rows, (int)cu_count(), st);
+                         hipStream_t st, bool exact = qmm::exact_forms()) {
+  if (type == qmm::T_Q6_K) return qmm::launch_gemm_q6k_skinny(t, k, p, rows, exact, st);
   return qmm::launch_gemm_q4k_skinny(t, k, p, rows, (int)cu_count(), st);
 }
 
@@ -601,17 +601,48 @@ int qmm_matvec(int type, const void* w, const void* xq, float* dst, int64_t ldd,
   return status_of(e);
 }
 
+// A product of the short-batch kernel with no room for its split slots
+// (qmm_matmul has none). A workgroup of it then walks a tile's whole K, which
+// takes 1.2 to 1.7 us a super-block, so where that leaves CUs idle the kernels
+// without slots take the product, as exactly: Q6_K past 32 rows the tiled GEMM,
+// otherwise the few-row kernel, 32 rows a launch, while the launches times their
+// rounds of the CUs (one per 4096 weight rows) are few. Uncut / here, us: Q4_K
+// 4096 x 14336 at 24 rows 99 / 20, 4096 x 4096 at 64 71 / 19, 8192 x 8192 at 96
+// 98 / 70; Q6_K 4096 x 14336 at 24 rows 135 / 34, 4096 x 4096 at 64 82 / 35;
+// but Q4_K 14336 x 4096 at 64 39 / 50, Q6_K at 24 40 / 49.
+int launch_mid_without_slots(int type, const void* w, int64_t n, int64_t k, const qmm::ActPlanes& p, int layout,
+                             int64_t rows, float* dst, int64_t ldd, hipStream_t st) {
+  if (qmm::gemm_kq_mid_splits(n, k, rows) > 1) {
+    if (type == qmm::T_Q6_K && rows >= qmm::gemm_q6k_min_rows() && qmm::gemm_q6k_fits(n, k, rows)) {
+      if (qmm::launch_gemm_q6k(w, n, k, p, rows, dst, ldd, st) != hipSuccess) return QMM_DEVICE_ERROR;
+      g_gemm_launches.fetch_add(1, std::memory_order_relaxed);
+      return QMM_OK;
+    }
+    const int64_t step = qmm::gemm_q4k_skinny_max_rows();
+    if ((rows + step - 1) / step * ((n + 4095) / 4096) <= (type == qmm::T_Q6_K ? 3 : 6)) {
+      for (int64_t r0 = 0; r0 < rows; r0 += step) {
+        const int64_t nr = rows - r0 < step ? rows - r0 : step;
+        if (launch_skinny(type, one_target(w, n, dst + r0 * ldd, ldd), k, qmm::act_rows(layout, p, k, r0), nr, st,
+                          true) != hipSuccess)
+          return QMM_DEVICE_ERROR;
+        g_gemm_launches.fetch_add(1, std::memory_order_relaxed);
+      }
+      return QMM_OK;
+    }
+  }
+  if (launch_mid(type, one_target(w, n, dst, ldd), k, p, rows, nullptr, 0, nullptr, st) != hipSuccess)
+    return QMM_DEVICE_ERROR;
+  g_gemm_launches.fetch_add(1, std::memory_order_relaxed);
+  return QMM_OK;
+}
+
 // One product from an activation already quantized into planes p (buffer
 // xq): the matrix-core kernels past the few-rows line, else the decode
 // kernels a chunk of at most matvec_max_rows() rows at a time.
 int launch_product(int type, const void* w, int64_t n, int64_t k, const void* xq, const qmm::ActPlanes& p,
                    int layout, int64_t rows, float* dst, int64_t ldd, hipStream_t st) {
-  if (mid_takes(type, w, xq, n, k, rows)) {
-    if (launch_mid(type, one_target(w, n, dst, ldd), k, p, rows, nullptr, 0, nullptr, st) != hipSuccess)
-      return QMM_DEVICE_ERROR;
-    g_gemm_launches.fetch_add(1, std::memory_order_relaxed);
-    return QMM_OK;
-  }
+  if (mid_takes(type, w, xq, n, k, rows))
+    return launch_mid_without_slots(type, w, n, k, p, layout, rows, dst, ldd, st);
   if (gemm_takes(type, w, xq, n, k, rows, st)) {
     if (launch_gemm(type, w, n, k, p, rows, dst, ldd, st) != hipSuccess) return QMM_DEVICE_ERROR;
     g_gemm_launches.fetch_add(1, std::memory_order_relaxed);

@@ -170,9 +170,9 @@ hipError_t launch_gemm_q4k_skinny(const MvTargets& t, int64_t k, const ActPlanes
                                   hipStream_t st);
 
 // Q6_K products of a few rows (gemm_q6k_skinny.hip): up to 32 activation
-// rows, targets as the stream kernels.
+// rows, targets as the stream kernels; exact: never the single-product form.
 bool gemm_q6k_skinny_fits(int64_t k, int64_t rows);
-hipError_t launch_gemm_q6k_skinny(const MvTargets& t, int64_t k, const ActPlanes& p, int64_t rows, int cus,
+hipError_t launch_gemm_q6k_skinny(const MvTargets& t, int64_t k, const ActPlanes& p, int64_t rows, bool exact,
                                   hipStream_t st);
 
 // The gate+up+GLU decode launch (mv_q4k.hip): Q4_K, 1-2 rows, k <= 8192;

@@ -1,7 +1,8 @@
 """Q4_K and Q6_K products of 17-128 rows (gemm_kq_mid.hip) against the CPU
 oracle: at the edges of its row tiles (32, 64, 96), of its row chunks
 (97, 129, 193 rows), of its 128-column tiles and of its K cut, and with the largest codes and
-scales a block can hold.
+scales a block can hold; and the kernels that take such a product where the
+workspace has no room for the slots of its cut.
 
 Bound: the super-block sums are exact integers and the min sums exact f32, so
 a result differs from the oracle's by f32 roundings only: per super-block
@@ -26,6 +27,15 @@ pytestmark = pytest.mark.gpu
 
 BOUND = 1e-5
 KERNEL = {qref.Q4_K: "launch_gemm_q4k_mid(", qref.Q6_K: "launch_gemm_q6k_mid("}
+
+
+def no_slots_kernel(t, n, rows):
+    """The kernel of a product that is cut, without room for its slots."""
+    if t == qref.Q6_K and rows > 32:
+        return "launch_gemm_q6k("
+    few = -(-rows // 32) * -(-n // 4096) <= (3 if t == qref.Q6_K else 6)
+    return ("launch_q6(" if t == qref.Q6_K else "launch_sk") if few else KERNEL[t]
+
 
 SHAPES = [  # (n, k, rows)
     (129, 1536, 33), (1, 1536, 40), (128, 1792, 64), (300, 4096, 65), (2048, 2048, 96), (255, 1536, 97),
@@ -53,7 +63,7 @@ def forward(t, qt, x, n, k, rows, ws_bytes=None):
 @pytest.mark.parametrize("t,n,k,rows", [(t, *s) for t in (qref.Q4_K, qref.Q6_K) for s in SHAPES]
                          + [(qref.Q6_K, *s) for s in CHUNKED]
                          + [(qref.Q4_K, 9000, 1792, 100), (qref.Q6_K, 9000, 4096, 90)])
-def test_against_the_oracle_and_the_same_bits_whatever_the_workspace(t, n, k, rows):
+def test_against_the_oracle_with_slots_and_without(t, n, k, rows):
     rng = np.random.default_rng(zlib.crc32(f"mid-{t}-{n}-{k}-{rows}".encode()))
     wq = qref.from_float(t, weights(rng, n, k))
     qt = QTensor.from_data(wq.tobytes(), (n, k), GgmlDType(t))
@@ -66,14 +76,20 @@ def test_against_the_oracle_and_the_same_bits_whatever_the_workspace(t, n, k, ro
     wdeq = qref.to_float(t, wq, n * k).reshape(n, k)
     err = normalised_error(y.cpu().numpy(), want, wdeq, x)
     assert err <= BOUND, err
-    # no room for the split slots: a workgroup adds a tile's splits in turn
+    # no room for the split slots: the kernels that need none, as exactly
     act = lib().qmm_act_bytes(_lib.ACT_Q8K, k, rows)
-    assert torch.equal(forward(t, qt, xt, n, k, rows, act)[0], y)
-    assert torch.equal(forward(t, qt, xt, n, k, rows, need - 1)[0], y) if need > act else True
+    other = no_slots_kernel(t, n, rows) if need > act else KERNEL[t]
+    small = forward(t, qt, xt, n, k, rows, act)[0]
+    assert other in lib().qmm_last_kernel().decode()
+    assert normalised_error(small.cpu().numpy(), want, wdeq, x) <= BOUND
+    assert torch.equal(small, y) or need > act
+    if need > act:
+        assert torch.equal(forward(t, qt, xt, n, k, rows, need - 1)[0], small)
     xq = quantize_act(xt, _lib.ACT_Q8K)
     out = torch.empty_like(y)
     assert lib().qmm_matmul(t, qt.data_.data_ptr(), xq.data_ptr(), out.data_ptr(), n, k, n, rows, stream()) == 0
-    assert torch.equal(out, y)
+    assert other in lib().qmm_last_kernel().decode()
+    assert torch.equal(out, small)
 
 
 LARGE = [  # up to 32 rows: the sizes the few-row kernels leave (n, k, rows, taken)
@@ -90,11 +106,17 @@ def test_large_weights_up_to_32_rows(t, n, k, rows, taken):
     print(f"t={t} n={n} k={k} rows={rows}", flush=True)
     y, need = forward(t, qt, xt, n, k, rows)
     assert (KERNEL[t] in lib().qmm_last_kernel().decode()) == taken
-    x, wq = xt.cpu().numpy(), qt.data_.cpu().numpy()
-    err = normalised_error(y.cpu().numpy(), qref.matmul(t, x, wq, n), qt.dequantize().cpu().numpy(), x)
+    x, wdeq = xt.cpu().numpy(), qt.dequantize().cpu().numpy()
+    want = qref.matmul(t, x, qt.data_.cpu().numpy(), n)
+    err = normalised_error(y.cpu().numpy(), want, wdeq, x)
     assert err <= (BOUND if taken or t == qref.Q4_K else 1e-3), err  # few-row Q6_K: its single-product form
     act = lib().qmm_act_bytes(_lib.ACT_Q8K, k, rows)
-    assert torch.equal(forward(t, qt, xt, n, k, rows, act)[0], y)
+    small = forward(t, qt, xt, n, k, rows, act)[0]
+    assert torch.equal(small, y) or taken
+    if taken:
+        kernel = lib().qmm_last_kernel().decode()
+        assert no_slots_kernel(t, n, rows) in kernel and "ONE = true" not in kernel
+        assert normalised_error(small.cpu().numpy(), want, wdeq, x) <= BOUND
 
 
 @pytest.mark.parametrize("rows", [33, 77, 128])
