@@ -453,14 +453,42 @@ void launch_fmt(const MidArgs& a, int units, hipStream_t st) {
 
 }  // namespace
 
-// The products this kernel takes. Up to 32 rows the few-row kernels, which
-// need no second launch, keep the smaller weights (this kernel against them at
-// 17 / 32 rows, one launch each: Q4_K 4096 x 4096 14.5 / 15.5 us against 10.7 /
-// 12.3, 8192 x 8192 23.6 / 24.5 against 22.7 / 27.9, 4096 x 14336 22.6 / 23.8
-// against 21.8 / 24.8, 14336 x 4096 22.5 / 23.5 against 23.9 / 29.2, 8192 x
-// 28672 57 / 61 against 64 / 79; Q6_K alike): it takes those of 14336 x 4096
-// values, below 24 rows only the wide ones and those over twice that.
-// Above 32 rows the tiled GEMMs keep rows of fewer than six super-blocks (1024
+// Up to 32 rows the few-row kernels, which need no second launch, keep what
+// fills their rounds of the CUs (4096 weight rows each). This kernel against
+// them, us, one weight at 17 / 24 / 32 rows:
+//   Q4_K  14336 x 4096   20.6 / 21.3 / 22.3 against 22.1 / 25.1 / 27.9
+//         28672 x 2048   17.5 / 17.7 / 18.2         33.1 / 36.9 / 38.8
+//         9216 x 4096    17.2 / 17.6 / 18.3         18.1 / 20.1 / 22.1
+//         12288 x 4096   20.2 / 20.3 / 21.2         18.6 / 21.1 / 22.9
+//         8192 x 8192    21.8 / 22.5 / 23.8         20.7 / 23.2 / 26.1
+//         5120 x 13824   23.3 / 24.3 / 25.3         30.7 / 34.7 / 39.5
+//         8192 x 7168    20.7 / 21.7 / 22.7         19.9 / 21.6 / 24.1
+//         8192 x 5120    17.2 / 18.0 / 18.8         15.8 / 17.4 / 18.6
+//         4096 x 13824   20.8 / 21.4 / 22.2         20.6 / 22.1 / 23.6
+//         1024 x 8192    13.3 / 13.8 / 14.0         13.5 / 14.9 / 15.9
+//         1024 x 12288   14.8 / 15.1 / 15.5         18.0 / 19.3 / 20.9
+//         2048 x 8192    14.1 / 14.6 / 15.3         14.0 / 15.1 / 15.9
+//         4096 x 4096    13.4 / 13.8 / 14.9         10.6 / 10.9 / 11.4
+//   Q6_K  9216 x 4096    22.4 / 22.6 / 23.4         27.6 / 29.3 / 30.5
+//         8192 x 7168    25.3 / 26.2 / 27.4         27.5 / 29.1 / 31.1
+//         4096 x 13824   25.1 / 26.0 / 26.8         25.4 / 26.3 / 27.1
+// Gate + up with the GLU gain more (Q4_K 13824 x 4096 at 24 rows 53 -> 29), q + k
+// + v sets less, and lose where the kernel takes only some of the weights (two
+// launches more: 8192, 2048, 2048 x 8192 at 24 rows 33.8 -> 36.8; 6144, 1024, 1024
+// x 6144 all here 23.3, all few-row 19.1). So 4097-8192 rows start at k = 7168 and 24
+// rows, and the narrow k and v go with their q (8192, 1024, 1024 x 8192 at 24 rows
+// all here 30.2, all few-row 32.5, apart 36.3).
+static bool few_rows_leave(int type, int64_t n, int64_t k, int64_t rows) {
+  constexpr int64_t kLong = (int64_t)4096 * 13824;
+  if (n * k >= 2 * kLong) return true;
+  if (n > 12288 || (type == T_Q6_K && n > 8192 && k < 7168)) return k >= 1536;
+  if (n <= 1024) return k >= (rows < 24 ? 10752 : 7168);
+  if (rows < 24) return false;
+  if (n > 8192) return k >= 3072;
+  return n > 4096 ? k >= 7168 : n * k >= kLong;
+}
+
+// The products this kernel takes. Above 32 rows the tiled GEMMs keep rows of fewer than six super-blocks (1024
 // x 1024 at 64 rows: 15.0 us against 14.7 here for Q4_K, 14.4 against 16.0 for
 // Q6_K) and, past 96 rows, the Q6_K products that fill them (14336 x 4096 at
 // 128 rows 44 us against 48); past 128 rows it takes the Q6_K products the
@@ -469,8 +497,7 @@ void launch_fmt(const MidArgs& a, int units, hipStream_t st) {
 bool gemm_kq_mid_fits(int type, int64_t n, int64_t k, int64_t rows) {
   const int64_t block = type == T_Q4_K ? 144 : type == T_Q6_K ? 210 : 0;
   if (rows <= 32) {
-    constexpr int64_t kLarge = (int64_t)14336 * 4096;
-    if (n * k < kLarge || (rows < 24 && n < 14336 && n * k < 2 * kLarge)) return false;
+    if (!few_rows_leave(type, n, k, rows)) return false;
   } else if (k < 1536) {
     return false;
   }

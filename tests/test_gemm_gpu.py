@@ -288,7 +288,7 @@ def test_matmul_from_a_quantized_activation_equals_forward(rows):
 # ---------------------------------------------------------------------------
 SKINNY_SHAPES = [  # (k, n, rows): past the 2 MiB line at 4-8 rows; ragged n; one and two 16-row tiles
     (4096, 2048, 4), (4096, 2050, 5), (8192, 1030, 8), (2048, 4100, 7), (256, 100, 9), (4096, 300, 16),
-    (14336, 64, 17), (1024, 500, 24), (8192, 129, 32),
+    (14336, 64, 17), (1024, 500, 24), (8192, 129, 32), (6144, 129, 32),
 ]
 
 

@@ -92,15 +92,20 @@ def test_against_the_oracle_with_slots_and_without(t, n, k, rows):
     assert torch.equal(out, small)
 
 
-LARGE = [  # up to 32 rows: the sizes the few-row kernels leave (n, k, rows, taken)
-    (14336, 4096, 17, True), (14335, 4096, 32, False), (4096, 14336, 24, True), (4096, 14336, 23, False),
-    (14340, 4096, 31, True), (8192, 14336, 17, True),
+LARGE = [  # up to 32 rows: the sizes the few-row kernels leave (n, k, rows, taken: of Q4_K, of Q6_K)
+    (12289, 1536, 17, True, True), (12288, 3072, 23, False, True), (8200, 3072, 24, True, True),
+    (8200, 2816, 24, False, True), (8200, 7168, 23, False, False), (8192, 4096, 32, False, False),
+    (4100, 7168, 24, True, True), (4100, 6912, 32, False, False), (4096, 7168, 32, False, False),
+    (1024, 7168, 24, True, True), (1025, 7168, 24, False, False), (1000, 10752, 17, True, True),
+    (1000, 10496, 23, False, False), (4096, 13824, 24, True, True), (4096, 13824, 23, False, False),
+    (14336, 4096, 17, True, True), (8192, 14336, 17, True, True),
 ]
 
 
 @pytest.mark.parametrize("t", [qref.Q4_K, qref.Q6_K], ids=["q4k", "q6k"])
-@pytest.mark.parametrize("n,k,rows,taken", LARGE)
-def test_large_weights_up_to_32_rows(t, n, k, rows, taken):
+@pytest.mark.parametrize("n,k,rows,q4k,q6k", LARGE)
+def test_large_weights_up_to_32_rows(t, n, k, rows, q4k, q6k):
+    taken = q4k if t == qref.Q4_K else q6k
     qt = QTensor.quantize(fill_normal(n * k, seed=n + k, std=0.02).reshape(n, k), GgmlDType(t))
     xt = fill_normal(rows * k, seed=rows).reshape(rows, k)
     print(f"t={t} n={n} k={k} rows={rows}", flush=True)
