@@ -104,8 +104,9 @@ int qmm_matvec(int type, const void *w, const void *xq, float *dst, int64_t ldd,
  * kernels up to qmm_matvec_max_rows() rows; for Q4_K and Q6_K the few-row
  * int8 matrix-core kernels from 4 rows on weights of 2 MiB or more and for
  * 9-32 rows, the exact short-batch kernel to 128 rows (from 17 for weights
- * of many or long rows, from 33 for k >= 1536; Q6_K to 256 rows
- * where k is no multiple of 2048), and the int8 matrix-core GEMMs past it;
+ * of many or long rows, from 33 for k >= 1536; Q6_K to 256 rows where k is
+ * no multiple of 2048, but not the sizes that its GEMM, as exact, runs
+ * faster), and the int8 matrix-core GEMMs past it;
  * for Q8_0, IQ4_NL and MXFP4 the int8 matrix-core GEMM from 9 rows. Nothing is
  * allocated, so a product that qmm_forward cuts along K into workspace slots
  * runs uncut here, at 17-128 rows on the few-row kernels (32 rows a launch) or

@@ -488,12 +488,43 @@ static bool few_rows_leave(int type, int64_t n, int64_t k, int64_t rows) {
   return n > 4096 ? k >= 7168 : n * k >= kLong;
 }
 
-// The products this kernel takes. Above 32 rows the tiled GEMMs keep rows of fewer than six super-blocks (1024
-// x 1024 at 64 rows: 15.0 us against 14.7 here for Q4_K, 14.4 against 16.0 for
-// Q6_K) and, past 96 rows, the Q6_K products that fill them (14336 x 4096 at
-// 128 rows 44 us against 48); past 128 rows it takes the Q6_K products the
-// single-pass GEMM leaves to the exact one (k no multiple of 2048): 4096 x
-// 11008 at 130 / 256 rows 45 / 75 us against 96 / 97.
+// Past 32 rows the tiled Q6_K GEMM, as exact, keeps what fills its tiles of 128
+// rows: this kernel against it, us, at 33 / 64 / 96 rows
+//   4096 x 1536    15.7 / 17.2 / 20.6 against 18.3 / 18.5 / 19.6
+//   8192 x 1536    16.7 / 19.5 / 23.8         18.3 / 18.6 / 19.7
+//   8192 x 2560    19.8 / 22.3 / 26.7         26.0 / 26.3 / 28.4
+//   14336 x 2048   22.4 / 25.5 / 30.9         22.6 / 22.8 / 24.7
+//   14336 x 2560   25.1 / 28.1 / 33.4         26.4 / 27.2 / 29.6
+//   14336 x 4096   31.8 / 34.8 / 41.6         38.3 / 38.7 / 42.5
+//   18944 x 1536   22.3 / 24.0 / 27.9         32.3 / 33.0 / 35.3
+// at 128 rows
+//   4096 x 4096 26.2 against 41.6, 8192 x 8192 55 / 77, 14336 x 8192 86 / 78,
+//   28672 x 8192 133 / 150, 65536 x 3072 116 / 93
+// and, where the single pass does not take them (k no multiple of 2048), at 160
+// / 256 rows
+//   1024 x 1536 18.4 / 20.2 against 20.0 / 20.2, 4096 x 1536 21.8 / 20.4 against
+//   20.2 / 20.5, 4096 x 2560 24.8 / 29.5 against 29.2 / 29.6, 4096 x 11008 48 / 77
+//   against 97 / 98, 8192 x 11008 78 / 131 against 98 / 100.
+static bool tiled_q6k_keeps(int64_t n, int64_t k, int64_t rows) {
+  if (rows <= 96) {
+    if (n <= 4096 || n > 16384) return false;
+    return k < (n <= 8192 ? (rows > 64 ? 2560 : 1536) : (rows > 64 ? 4096 : 2560));
+  }
+  if (rows > 192) return n > 4096 || k < 4096;
+  if (n <= 4096) return rows > 128 && n > 2048 && k < 2560;
+  return k < 8192 || (rows <= 128 && ((n > 8192 && n <= 16384) || n > 32768));
+}
+
+// The products this kernel takes. Above 32 rows the tiled GEMMs keep rows of
+// fewer than six super-blocks: of k = 1024 weights of 1024 to 8192 rows take
+// 0.89-1.08 (Q4_K) and 1.02-1.22 times (Q6_K) as long here at 33-64 rows,
+// 1.05-1.39 and 1.18-1.40 at 65-96, and a launch more of host time; from k = 1536
+// 0.71-0.93 and 0.82-1.05. Q4_K keeps past that to 128 rows though the tiled
+// (two-pass) GEMM is faster for some: weights of more than 16384 rows at 65-96 rows
+// 1.04-1.2 times, at 97-128 1.15-1.25 (65536 rows 1.5: 92 us against 60 at k =
+// 3072), and k below 3072 at 65-96 rows 1.05-1.3 (14336 x 1536 26.5 against 20.4):
+// it rounds the min sums to f16 (9e-4 of the result's norm where this kernel is
+// within 1e-7).
 bool gemm_kq_mid_fits(int type, int64_t n, int64_t k, int64_t rows) {
   const int64_t block = type == T_Q4_K ? 144 : type == T_Q6_K ? 210 : 0;
   if (rows <= 32) {
@@ -501,8 +532,8 @@ bool gemm_kq_mid_fits(int type, int64_t n, int64_t k, int64_t rows) {
   } else if (k < 1536) {
     return false;
   }
-  if (type == T_Q6_K && rows > 96 && n > 4096 && k < 8192) return false;
-  if (rows > 128 && (type != T_Q6_K || k % 2048 == 0 || rows > 256 || (rows > 192 && k < 4096))) return false;
+  if (type == T_Q6_K && rows > 32 && tiled_q6k_keeps(n, k, rows)) return false;
+  if (rows > 128 && (type != T_Q6_K || k % 2048 == 0 || rows > 256)) return false;
   // 32-bit byte offsets inside the kernel
   return block != 0 && rows >= kMidMinRows && k % 256 == 0 && n * (k / 256) * block + 16 < ((int64_t)1 << 31) &&
          256 * k < ((int64_t)1 << 31) && n * rows < ((int64_t)1 << 31);

@@ -124,6 +124,32 @@ def test_large_weights_up_to_32_rows(t, n, k, rows, q4k, q6k):
         assert normalised_error(small.cpu().numpy(), want, wdeq, x) <= BOUND
 
 
+LINES = [  # past 32 rows: the Q6_K products the tiled GEMM keeps (n, k, rows, taken here)
+    (4096, 1536, 96, True), (8192, 1536, 64, True), (8192, 1536, 65, False), (4100, 2560, 96, True),
+    (8200, 2304, 64, False), (8200, 2560, 33, True), (16384, 3840, 65, False), (16384, 4096, 96, True),
+    (16390, 1536, 96, True), (4096, 1536, 128, True), (8192, 8192, 97, True), (8200, 8192, 97, False),
+    (16390, 8192, 128, True), (32780, 8192, 97, False), (4096, 2304, 129, False),
+    (2048, 2304, 129, True), (4096, 2560, 192, True), (4100, 8448, 192, True), (4096, 4352, 193, True), (4100, 8448, 193, False),
+]
+
+
+@pytest.mark.parametrize("n,k,rows,taken", LINES)
+def test_q6k_lines_to_the_tiled_gemm(n, k, rows, taken):
+    """Each side of every line, against the oracle at the first, last and 64
+    weight rows between."""
+    qt = QTensor.quantize(fill_normal(n * k, seed=n + k, std=0.02).reshape(n, k), GgmlDType.Q6K)
+    xt = fill_normal(rows * k, seed=rows).reshape(rows, k)
+    print(f"n={n} k={k} rows={rows}", flush=True)
+    y = QMatMul(qt).forward(xt)
+    assert (KERNEL[qref.Q6_K] if taken else "launch_gemm_q6k(") in lib().qmm_last_kernel().decode()
+    some = np.unique(np.linspace(0, n - 1, 66).astype(np.int64))
+    wq = np.ascontiguousarray(qt.data_.reshape(-1)[: n * k // 256 * 210].cpu().numpy().reshape(n, -1)[some]).reshape(-1)
+    x = xt.cpu().numpy()
+    want = qref.matmul(qref.Q6_K, x, wq, len(some))
+    wdeq = qref.to_float(qref.Q6_K, wq, len(some) * k).reshape(len(some), k)
+    assert normalised_error(y[:, torch.from_numpy(some).cuda()].cpu().numpy(), want, wdeq, x) <= BOUND
+
+
 @pytest.mark.parametrize("rows", [33, 77, 128])
 def test_shared_products_keep_each_weights_bits(rows):
     """Five weights (two launches) of which some are cut and some are not."""
