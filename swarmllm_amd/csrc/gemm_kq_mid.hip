@@ -31,7 +31,7 @@
 //   - The activation codes of a super-block (32 MT rows x 256 B, pieces
 //     XOR-swizzled by row) reach LDS by direct copies, one super-block ahead,
 //     double-buffered; the code sums (as f16) and dy through registers.
-// //   - A wave's raw weight bytes weight bytes (32 rows' blocks as their aligned 16-byte
+//   - A wave's weight bytes (32 rows' blocks as their aligned 16-byte
 //     pieces) are loaded one super-block ahead into registers, consecutive
 //     lanes on consecutive pieces, and written to the wave's own LDS slot
 //     when the current super-block is done; lanes read their row back.
@@ -41,8 +41,8 @@
 // their outputs are never stored.
 //
 // Measured at 77 rows (an 8B layer, slots added in): q + k + v 24 us, o 19,
-// gate + up with its GLU 45, down 34; at 21 rows 15 / 13 / 28 / 26 (the
-// two-row-tile few-row kernels before: 13 / 9 / 54 / 25). At 21 rows gate + up
+// gate + up with its GLU 45, down 34; at 21 rows gate + up with its GLU 28 (the
+// two-row-tile few-row kernel before: 54; it keeps the others). At 21 rows gate + up
 // reads HBM at 4.9 TB/s, 1.5 x its weight bytes (the 64-byte sector at each
 // 144-byte block's edges is fetched twice); at 77 the vector unit is busy 41%
 // and the matrix cores 30% of the time. The weight loads are nontemporal:
@@ -458,6 +458,8 @@ void launch_fmt(const MidArgs& a, int units, hipStream_t st) {
 // them, us, one weight at 17 / 24 / 32 rows:
 //   Q4_K  14336 x 4096   20.6 / 21.3 / 22.3 against 22.1 / 25.1 / 27.9
 //         28672 x 2048   17.5 / 17.7 / 18.2         33.1 / 36.9 / 38.8
+//         28672 x 512     9.7 /  9.5 /  9.8         21.5 / 24.4 / 24.6
+//         14336 x 1024   12.6 / 13.0 / 13.8         11.7 / 12.5 / 12.9
 //         9216 x 4096    17.2 / 17.6 / 18.3         18.1 / 20.1 / 22.1
 //         12288 x 4096   20.2 / 20.3 / 21.2         18.6 / 21.1 / 22.9
 //         8192 x 8192    21.8 / 22.5 / 23.8         20.7 / 23.2 / 26.1
@@ -480,7 +482,7 @@ void launch_fmt(const MidArgs& a, int units, hipStream_t st) {
 // all here 30.2, all few-row 32.5, apart 36.3).
 static bool few_rows_leave(int type, int64_t n, int64_t k, int64_t rows) {
   constexpr int64_t kLong = (int64_t)4096 * 13824;
-  if (n * k >= 2 * kLong) return true;
+  if (n > 16384 || n * k >= 2 * kLong) return true;
   if (n > 12288 || (type == T_Q6_K && n > 8192 && k < 7168)) return k >= 1536;
   if (n <= 1024) return k >= (rows < 24 ? 10752 : 7168);
   if (rows < 24) return false;
@@ -527,6 +529,7 @@ static bool tiled_q6k_keeps(int64_t n, int64_t k, int64_t rows) {
 // within 1e-7).
 bool gemm_kq_mid_fits(int type, int64_t n, int64_t k, int64_t rows) {
   const int64_t block = type == T_Q4_K ? 144 : type == T_Q6_K ? 210 : 0;
+  if (block == 0 || rows < kMidMinRows) return false;
   if (rows <= 32) {
     if (!few_rows_leave(type, n, k, rows)) return false;
   } else if (k < 1536) {
@@ -535,8 +538,8 @@ bool gemm_kq_mid_fits(int type, int64_t n, int64_t k, int64_t rows) {
   if (type == T_Q6_K && rows > 32 && tiled_q6k_keeps(n, k, rows)) return false;
   if (rows > 128 && (type != T_Q6_K || k % 2048 == 0 || rows > 256)) return false;
   // 32-bit byte offsets inside the kernel
-  return block != 0 && rows >= kMidMinRows && k % 256 == 0 && n * (k / 256) * block + 16 < ((int64_t)1 << 31) &&
-         256 * k < ((int64_t)1 << 31) && n * rows < ((int64_t)1 << 31);
+  return k % 256 == 0 && n * (k / 256) * block + 16 < ((int64_t)1 << 31) && 256 * k < ((int64_t)1 << 31) &&
+         n * rows < ((int64_t)1 << 31);
 }
 
 // K ranges of one weight's product, from its own shape (so a weight's bits do
