@@ -107,8 +107,9 @@ int qmm_matvec(int type, const void *w, const void *xq, float *dst, int64_t ldd,
  * of many or long rows, from 33 for k >= 1536; Q6_K to 256 rows where k is
  * no multiple of 2048, but not the sizes that its GEMM, as exact, runs
  * faster), and the int8 matrix-core GEMMs past it;
- * for Q8_0, IQ4_NL and MXFP4 the int8 matrix-core GEMM from 9 rows. Nothing is
- * allocated, so a product that qmm_forward cuts along K into workspace slots
+ * for Q8_0, IQ4_NL and MXFP4 the int8 matrix-core GEMM from 9 rows, whose f32
+ * sums run in one to eight K ranges by rows and n (a row's last bits can depend
+ * on both, past 8 rows). Nothing is allocated, so a product that qmm_forward cuts along K into workspace slots
  * runs uncut here, at 17-128 rows on the few-row kernels (32 rows a launch) or
  * the Q6_K GEMM where they are faster: 1.1 to 3 times qmm_forward's time.
  * The SWARMLLM_QMATMUL_MMQ switches below move these lines. Replaces
@@ -143,7 +144,8 @@ int qmm_mmq_captured(void);
  * feed the matrix cores a rounded product of a code and its sub-block scale
  * (normalised error up to about 1e-3, inside the 2e-3 bound): the
  * single-pass Q4_K and Q6_K GEMMs (from 129 rows) and the few-row Q6_K
- * kernel's single-product form (k >= 2048, from the few-rows line to 16 rows), so a product's bits
+ * kernel's single-product form (k >= 2048, from the few-rows line to 32 rows where
+ * the short-batch kernel does not take the weight), so a product's bits
  * can depend on the row count of its batch (1-2 rows are always exact). With
  * it every row count sums exact int32 products, at the exact kernels' speed.
  * qmm_exact_forms: 1 when the switch is on. */
